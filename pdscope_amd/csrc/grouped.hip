@@ -43,12 +43,20 @@ typedef __attribute__((address_space(1))) const void g_void_t;
 
 // One wave-wide direct-to-LDS load: lane l's 16 bytes at src land at
 // dst + 16 l (dst is wave-uniform), bypassing the registers.  AUX is the
-// cache-policy field: kDeviceScope (sc1) makes the load device-coherent, so
-// it is served by the L2 without allocating in the CU's vector L1.  Weight
-// tiles are read once per CU and use it (measured: about 10% faster grouped
-// launches at T=4096 than with L1 allocation, while nt, the streaming hint,
-// was slower); activation tiles keep the default.
+// cache-policy field.  kDeviceScope (sc1) makes the load device-coherent, so
+// it is served by the L2 without allocating in the CU's vector L1; kStream
+// (nt) marks the lines as not to be kept.  A weight tile is read once per
+// m-tile of its expert: where the expert has one m-tile nothing will ask for
+// it again, and streaming reads run at 7.0 TB/s against 6.3 and leave the L2
+// to the activations; where it has more, the m-tiles read it at about the
+// same time and the second should hit the L2.  Chosen per tile, against sc1
+// throughout: Qwen shape T=201 gate/up 143 -> 128 us, down 79 -> 71; T=512
+// 145 -> 135 and 83 -> 76; T=4096 (about half the experts have two tiles)
+// 289 -> 284 and 167 -> 160; DeepSeek-V2-Lite shape T=1304 down 95 -> 82.
+// nt throughout: T=512 with Zipf routing 159 against 148, T=4096 301.
+// Activation tiles keep the default policy.
 constexpr int kDeviceScope = 16;
+constexpr int kStream = 2;
 template <int AUX = 0>
 __device__ __forceinline__ void load_lds16(const uint16_t *src, uint8_t *dst) {
     __builtin_amdgcn_global_load_lds((g_void_t *)(uintptr_t)src, (lds_void_t *)(uint32_t)(uintptr_t)dst, 16, 0, AUX);
@@ -223,6 +231,8 @@ __global__ __launch_bounds__(64 * WM * WN, OCC == 1 ? 1 : OCC * WM * WN / 4) voi
     };
     const uint8_t *const a_base = reinterpret_cast<const uint8_t *>(a_src);
     const uint8_t *const b_base = reinterpret_cast<const uint8_t *>(base);
+    const bool one_tile = row_end - offsets[e] <= BM;  // no other m-tile reads these weights
+    const int KT = K / BK;
     auto issue_a = [&](int kt) __attribute__((always_inline)) {
         uint8_t *st = ring_a + (kt % SA) * ASTAGE;
         const uint8_t *b = a_base + kt * (BK * 2);
@@ -243,15 +253,20 @@ __global__ __launch_bounds__(64 * WM * WN, OCC == 1 ? 1 : OCC * WM * WN / 4) voi
                 }
             }
     };
-    auto issue_b = [&](int kt) __attribute__((always_inline)) {
+    auto issue_b_as = [&](int kt, auto aux) __attribute__((always_inline)) {
         uint8_t *st = ring_b + (kt % SB) * BSTAGE;
         const uint8_t *b = b_base + kt * (BK * 2);
 #pragma unroll
         for (int q = 0; q < BL; ++q) {
             uint32_t o = b_lane;
             opaque(o);
-            load_lds16<kDeviceScope>(reinterpret_cast<const uint16_t *>(b + b_row0(q) + o), st + (wb + NWB * q) * 1024);
+            load_lds16<decltype(aux)::value>(reinterpret_cast<const uint16_t *>(b + b_row0(q) + o),
+                                             st + (wb + NWB * q) * 1024);
         }
+    };
+    auto issue_b = [&](int kt) __attribute__((always_inline)) {
+        if (one_tile) issue_b_as(kt, std::integral_constant<int, kStream>{});
+        else issue_b_as(kt, std::integral_constant<int, kDeviceScope>{});
     };
 
     const int wm = wave / WN, wn = wave % WN;
@@ -277,7 +292,6 @@ __global__ __launch_bounds__(64 * WM * WN, OCC == 1 ? 1 : OCC * WM * WN / 4) voi
     const int live_blocks = (row_end - m0 + 31) / 32;
     const int mb_live = __builtin_amdgcn_readfirstlane(
         ILV ? min(MB, max(0, (live_blocks - wm + WM - 1) / WM)) : min(MB, max(0, (row_end - m0 - wm * TM + 31) / 32)));
-    const int KT = K / BK;
     // Software-pipelined K loop.  Slot kt % SA of the A ring and kt % SB of
     // the B ring hold stage kt; the stages up to kt+SA-1 / kt+SB-1 are in
     // flight while stage kt is consumed, and the LDS reads of stage kt+1
