@@ -72,6 +72,14 @@ __device__ __forceinline__ uint4 ld_nt(const void *p) {
     return make_uint4(v.x, v.y, v.z, v.w);
 }
 
+// 16-byte store that writes through the L2 as it is made (sc1, device
+// scope): results no later block of the launch reads.  Plain stores stay in
+// the L2s, which write back what they hold while the kernel ends.
+__device__ __forceinline__ void st_through(void *p, uint4 v) {
+    const u32x4_t d = {v.x, v.y, v.z, v.w};
+    asm volatile("global_store_dwordx4 %0, %1, off sc1" ::"v"(p), "v"(d) : "memory");
+}
+
 // plain 16-byte global load
 __device__ __forceinline__ uint4 ld_g(const void *p) {
     u32x4_t v = *gptr(p);

@@ -329,7 +329,9 @@ __global__ __launch_bounds__(64 * WM * WN, OCC == 1 ? 1 : OCC * WM * WN / 4) voi
                 for (int i = 0; i < L; ++i)
 #pragma unroll
                     for (int j = 0; j < NB; ++j)
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[buf][kk][i], bfr[buf][kk][j],
+                        // weights as the first operand: a lane then holds one
+                        // activation row and four weight rows in a row (epilogue)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bfr[buf][kk][j], af[buf][kk][i],
                                                                             acc[i][j], 0, 0, 0);
         };
         // prologue: every ring filled, stage 0 landed
@@ -449,32 +451,52 @@ __global__ __launch_bounds__(64 * WM * WN, OCC == 1 ? 1 : OCC * WM * WN / 4) voi
         }
     }
 
-    // ---- epilogue: lane holds column (lane & 31), rows (r/4)*8 + (lane/32)*4 + r%4
+    // ---- epilogue.  A lane holds row (lane & 31) of each 32x32 block and its
+    // columns (r/4)*8 + (lane/32)*4 + r%4, i.e. four groups of four columns.
+    // The tile goes through LDS (the ring is free now) and out in 16-byte
+    // stores along whole rows, written through.  Against 2-byte stores straight from the
+    // accumulators: DeepSeek-V2-Lite shape T=1304 gate/up 167 -> 148 us, down 82 ->
+    // 74; Qwen shape T=512 down 76 -> 71, T=4096 down 167 -> 158; whole layers
+    // T=512 240 -> 231, T=1304 374 -> 354.  (Row-wise stores without the
+    // write-through gave 161 / 82 / 76 / 161.)  A staged row is 16 bytes longer than a multiple of
+    // the 256-byte bank line: the 16 rows of a quarter-wave write land in
+    // distinct banks.
+    constexpr int CO = GATEUP ? BN / 2 : BN;  // output columns of the tile
+    constexpr int OB = CO * 2 + 16;           // bytes of a staged row
+    static_assert(BM * OB <= SA * ASTAGE + SB * BSTAGE, "staged output fits the ring");
+    __syncthreads();  // every wave has read its last stage
 #pragma unroll
     for (int i = 0; i < MB; ++i) {
+        if (m0 + rblk(i) >= row_end) continue;  // wave-uniform
+        uint8_t *const srow = smem + (rblk(i) + lrow) * OB + (wn * (GATEUP ? TN / 2 : TN) + lhalf * 4) * 2;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const int row = m0 + rblk(i) + (r >> 2) * 8 + lhalf * 4 + (r & 3);
-            if (row >= row_end) continue;
-            if (GATEUP) {
+        for (int j = 0; j < (GATEUP ? NB / 2 : NB); ++j)
 #pragma unroll
-                for (int j = 0; j < NB / 2; ++j) {
-                    const int col = n0 + wn * (TN / 2) + j * 32 + lrow;
-                    // g and u rounded by one conversion
-                    const uint32_t gu = f2bf2_hw(acc[i][j][r], acc[i][j + NB / 2][r]);
-                    const float g = __uint_as_float(gu << 16);
-                    const float u = __uint_as_float(gu & 0xffff0000u);
-                    const float a = bf16_round_hw(silu_fast(g));
-                    out[(size_t)row * I + col] = (uint16_t)f2bf_hw(a * u);
+            for (int q = 0; q < 4; ++q) {
+                uint32_t w[2];
+#pragma unroll
+                for (int p = 0; p < 2; ++p) {
+                    const int r = q * 4 + p * 2;
+                    if constexpr (GATEUP) {
+                        const uint32_t g = f2bf2_hw(acc[i][j][r], acc[i][j][r + 1]);
+                        const uint32_t u = f2bf2_hw(acc[i][j + NB / 2][r], acc[i][j + NB / 2][r + 1]);
+                        const uint32_t a = f2bf2_hw(silu_fast(lo_bf(g)), silu_fast(hi_bf(g)));
+                        w[p] = f2bf2_hw(lo_bf(a) * lo_bf(u), hi_bf(a) * hi_bf(u));
+                    } else {
+                        w[p] = f2bf2_hw(acc[i][j][r], acc[i][j][r + 1]);
+                    }
                 }
-            } else {
-#pragma unroll
-                for (int j = 0; j < NB; ++j) {
-                    const int col = n0 + wn * TN + j * 32 + lrow;
-                    out[(size_t)row * H + col] = (uint16_t)f2bf_hw(acc[i][j][r]);
-                }
+                *reinterpret_cast<uint2 *>(srow + (j * 32 + q * 8) * 2) = make_uint2(w[0], w[1]);
             }
-        }
+    }
+    __syncthreads();
+    constexpr int CH = CO / 8;  // 16-byte chunks per row
+    const int ldo = GATEUP ? I : H;
+    const int chunks = min(BM, row_end - m0) * CH;
+    for (int c = tid; c < chunks; c += 64 * NW) {
+        const int row = c / CH, ch = c % CH;
+        st_through(out + (size_t)(m0 + row) * ldo + n0 + ch * 8,
+                   *reinterpret_cast<const uint4 *>(smem + row * OB + ch * 16));
     }
 }
 
@@ -520,9 +542,23 @@ int grouped_entry(int phase, const void *x, const int32_t *perm_token, const int
     const uint16_t *xp = (const uint16_t *)x;
     const uint16_t *const *sp = (const uint16_t *const *)slots;
     switch (block_m) {
-    case 32:
-        return launch_grouped<32, 256, 64, 1, 4, 4, 4>(phase, xp, perm_token, offsets, sel, nsel, tile_start, max_tiles, sp,
-                                                H, I, (uint16_t *)h_ws, (uint16_t *)y, s);
+    case 32: {
+        // down (K = I, a short K loop): two workgroups of 128 columns per CU, so
+        // that one's ring fill and epilogue overlap the other's loads (T=201:
+        // 71 -> 67 us, T=17: 46.8 -> 44.5); gate/up is faster on 256 columns
+        // and a CU of its own (T=201: 128 us against 136 at two per CU)
+        if (H % 256) return fail(kEInval, "grouped: H must divide by 256");
+        int rc = kOk;
+        if (phase & 1)
+            rc = launch_grouped<32, 256, 64, 1, 4, 4, 4, false, 1>(1, xp, perm_token, offsets, sel, nsel, tile_start,
+                                                                   max_tiles, sp, H, I, (uint16_t *)h_ws,
+                                                                   (uint16_t *)y, s);
+        if (rc == kOk && (phase & 2))
+            rc = launch_grouped<32, 128, 64, 1, 4, 4, 4, false, 2, 2>(2, xp, perm_token, offsets, sel, nsel, tile_start,
+                                                                      max_tiles, sp, H, I, (uint16_t *)h_ws,
+                                                                      (uint16_t *)y, s);
+        return rc;
+    }
     case 64: {
         // gate/up: split load roles, 3 + 4 stages, one workgroup per CU; down
         // (K = I, a short K loop): every wave loads both operands, 2 + 2
