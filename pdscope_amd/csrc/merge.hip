@@ -19,12 +19,58 @@
 
 namespace pd {
 
-// KM > 0: k <= KM, and the k row indices, weights and rows of a thread are
-// loaded before the first is used (two memory latencies per output chunk
-// instead of 2k); KM == 0: any k, one slot at a time.  The fp32
-// accumulation is the same in both: slot order, one rounding.
-// ORDERED: the reference's arithmetic instead -- rows in ascending grouped
-// row, acc = bf16(acc + bf16(w * y)) per row, add_in added last.
+// One output chunk of eight columns in either arithmetic.
+template <bool ORDERED>
+struct MergeAcc {
+    float a[8];
+    __device__ __forceinline__ void set(uint4 v) {
+        a[0] = lo_bf(v.x); a[1] = hi_bf(v.x); a[2] = lo_bf(v.y); a[3] = hi_bf(v.y);
+        a[4] = lo_bf(v.z); a[5] = hi_bf(v.z); a[6] = lo_bf(v.w); a[7] = hi_bf(v.w);
+    }
+    __device__ __forceinline__ void zero() {
+#pragma unroll
+        for (int q = 0; q < 8; ++q) a[q] = 0.0f;
+    }
+    // two columns: a = bf16(a + p)
+    __device__ __forceinline__ void round_add(int q, float p0, float p1) {
+        const uint32_t r = f2bf2_hw(a[q] + p0, a[q + 1] + p1);
+        a[q] = lo_bf(r);
+        a[q + 1] = hi_bf(r);
+    }
+    __device__ __forceinline__ void add(float w, uint4 v) {
+        const uint32_t x[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            if constexpr (ORDERED) {
+                const uint32_t p = f2bf2_hw(w * lo_bf(x[q]), w * hi_bf(x[q]));
+                round_add(2 * q, lo_bf(p), hi_bf(p));
+            } else {
+                a[2 * q] = __builtin_fmaf(w, lo_bf(x[q]), a[2 * q]);
+                a[2 * q + 1] = __builtin_fmaf(w, hi_bf(x[q]), a[2 * q + 1]);
+            }
+        }
+    }
+    __device__ __forceinline__ void add_last(uint4 v) {
+        round_add(0, lo_bf(v.x), hi_bf(v.x));
+        round_add(2, lo_bf(v.y), hi_bf(v.y));
+        round_add(4, lo_bf(v.z), hi_bf(v.z));
+        round_add(6, lo_bf(v.w), hi_bf(v.w));
+    }
+    __device__ __forceinline__ uint4 result() const {
+        return make_uint4(f2bf2_hw(a[0], a[1]), f2bf2_hw(a[2], a[3]), f2bf2_hw(a[4], a[5]), f2bf2_hw(a[6], a[7]));
+    }
+};
+
+// k <= KM: one wave per token and 64 output chunks (512 columns).  The
+// token's k row indices and weights are the same for the whole wave: lane s
+// holds slot s, the k values become scalars by lane reads, and all k rows of
+// a lane's chunk are loaded before the first is added.
+// Bound by the bytes of y.  ORDERED (rows in ascending grouped row, acc =
+// bf16(acc + bf16(w * y)) per row, add_in added last): each lane ranks its
+// slot against the others (k compares) and one lane push sorts them; a loop
+// over all k for each next row in every thread took 71 us at T=4096, k=8,
+// H=2048 (about 36 now, 31 for the fp32 sum), and the roundings in integer
+// arithmetic more than the loads (now the hardware's pair conversion).
 template <int KM, bool ORDERED>
 __global__ __launch_bounds__(256) void merge_kernel(const uint16_t *__restrict__ y,
                                                     const int32_t *__restrict__ row_of,
@@ -32,72 +78,66 @@ __global__ __launch_bounds__(256) void merge_kernel(const uint16_t *__restrict__
                                                     const uint16_t *__restrict__ add_in,
                                                     uint16_t *__restrict__ out) {
     const int CH = H >> 3;
+    const int groups = (CH + 63) >> 6;
+    const int lane = lane_id();
+    const int64_t total = (int64_t)T * groups;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    for (int64_t item = (int64_t)blockIdx.x * 4 + wave; item < total; item += (int64_t)gridDim.x * 4) {
+        const int t = (int)(item / groups), g = (int)(item - (int64_t)t * groups);
+        const int c = g * 64 + lane;
+        const bool live = c < CH;
+        const int cc = live ? c : CH - 1;
+        const size_t s0 = (size_t)t * k + min(lane, k - 1);
+        int row = row_of[s0];
+        int wb = w[s0];
+        uint4 addv = make_uint4(0, 0, 0, 0);
+        if (add_in) addv = reinterpret_cast<const uint4 *>(add_in + (size_t)t * H)[cc];
+        if constexpr (ORDERED) {
+            int rank = 0;
+#pragma unroll
+            for (int s = 0; s < KM; ++s)
+                if (s < k) {
+                    const int o = __builtin_amdgcn_readlane(row, s);
+                    rank += (o < row) | ((o == row) & (s < lane));
+                }
+            // lane s's slot to lane `rank`; lanes past k keep to themselves
+            const int dst = (lane < k ? rank : lane) * 4;
+            row = __builtin_amdgcn_ds_permute(dst, row);
+            wb = __builtin_amdgcn_ds_permute(dst, wb);
+        }
+        uint4 v[KM];
+#pragma unroll
+        for (int s = 0; s < KM; ++s)
+            if (s < k)
+                v[s] = reinterpret_cast<const uint4 *>(y + (size_t)__builtin_amdgcn_readlane(row, s) * H)[cc];
+        MergeAcc<ORDERED> acc;
+        if (!ORDERED && add_in) acc.set(addv);
+        else acc.zero();
+#pragma unroll
+        for (int s = 0; s < KM; ++s)
+            if (s < k) acc.add(bf2f((uint32_t)__builtin_amdgcn_readlane(wb, s)), v[s]);
+        if (ORDERED && add_in) acc.add_last(addv);
+        if (live) reinterpret_cast<uint4 *>(out + (size_t)t * H)[c] = acc.result();
+    }
+}
+
+// any k, one thread per chunk, one slot at a time
+template <bool ORDERED>
+__global__ __launch_bounds__(256) void merge_any_kernel(const uint16_t *__restrict__ y,
+                                                        const int32_t *__restrict__ row_of,
+                                                        const uint16_t *__restrict__ w, int T, int k, int H,
+                                                        const uint16_t *__restrict__ add_in,
+                                                        uint16_t *__restrict__ out) {
+    const int CH = H >> 3;
     const int64_t total = (int64_t)T * CH;
     for (int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; idx < total;
          idx += (int64_t)gridDim.x * blockDim.x) {
         const int t = (int)(idx / CH), c = (int)(idx - (int64_t)t * CH);
-        float acc[8];
-        if (ORDERED) {
-#pragma unroll
-            for (int q = 0; q < 8; ++q) acc[q] = 0.0f;
-        } else if (add_in) {
-            const uint4 v = reinterpret_cast<const uint4 *>(add_in + (size_t)t * H)[c];
-            acc[0] = lo_bf(v.x); acc[1] = hi_bf(v.x); acc[2] = lo_bf(v.y); acc[3] = hi_bf(v.y);
-            acc[4] = lo_bf(v.z); acc[5] = hi_bf(v.z); acc[6] = lo_bf(v.w); acc[7] = hi_bf(v.w);
-        } else {
-#pragma unroll
-            for (int q = 0; q < 8; ++q) acc[q] = 0.0f;
-        }
-        auto add = [&](float ws, uint4 v) __attribute__((always_inline)) {
-            if constexpr (ORDERED) {
-                const float yv[8] = {lo_bf(v.x), hi_bf(v.x), lo_bf(v.y), hi_bf(v.y),
-                                     lo_bf(v.z), hi_bf(v.z), lo_bf(v.w), hi_bf(v.w)};
-#pragma unroll
-                for (int q = 0; q < 8; ++q) acc[q] = bf16_round(acc[q] + bf16_round(ws * yv[q]));
-                return;
-            }
-            acc[0] = __builtin_fmaf(ws, lo_bf(v.x), acc[0]);
-            acc[1] = __builtin_fmaf(ws, hi_bf(v.x), acc[1]);
-            acc[2] = __builtin_fmaf(ws, lo_bf(v.y), acc[2]);
-            acc[3] = __builtin_fmaf(ws, hi_bf(v.y), acc[3]);
-            acc[4] = __builtin_fmaf(ws, lo_bf(v.z), acc[4]);
-            acc[5] = __builtin_fmaf(ws, hi_bf(v.z), acc[5]);
-            acc[6] = __builtin_fmaf(ws, lo_bf(v.w), acc[6]);
-            acc[7] = __builtin_fmaf(ws, hi_bf(v.w), acc[7]);
-        };
-        if constexpr (KM > 0) {
-            int r[KM];
-            float ws[KM];
-#pragma unroll
-            for (int s = 0; s < KM; ++s) {
-                r[s] = s < k ? row_of[(size_t)t * k + s] : 0;
-                ws[s] = s < k ? bf2f(w[(size_t)t * k + s]) : 0.0f;
-            }
-            if constexpr (ORDERED) {
-                // ascending grouped row (= ascending expert id): compare-exchange
-                // passes over the live entries, indices static after unrolling
-#pragma unroll
-                for (int a = 1; a < KM; ++a)
-#pragma unroll
-                    for (int b = KM - 1; b >= a; --b)
-                        if (b < k && r[b - 1] > r[b]) {
-                            const int tr = r[b];
-                            r[b] = r[b - 1];
-                            r[b - 1] = tr;
-                            const float tw = ws[b];
-                            ws[b] = ws[b - 1];
-                            ws[b - 1] = tw;
-                        }
-            }
-            uint4 v[KM];
-#pragma unroll
-            for (int s = 0; s < KM; ++s)
-                if (s < k) v[s] = reinterpret_cast<const uint4 *>(y + (size_t)r[s] * H)[c];
-#pragma unroll
-            for (int s = 0; s < KM; ++s)
-                if (s < k) add(ws[s], v[s]);
-        } else if constexpr (ORDERED) {
-            // any k: the next larger grouped row each round
+        MergeAcc<ORDERED> acc;
+        if (!ORDERED && add_in) acc.set(reinterpret_cast<const uint4 *>(add_in + (size_t)t * H)[c]);
+        else acc.zero();
+        if constexpr (ORDERED) {
+            // the next larger grouped row each round
             int prev = -1;
             for (int n = 0; n < k; ++n) {
                 int best = 0x7fffffff, bs = 0;
@@ -109,27 +149,16 @@ __global__ __launch_bounds__(256) void merge_kernel(const uint16_t *__restrict__
                     }
                 }
                 prev = best;
-                add(bf2f(w[(size_t)t * k + bs]), reinterpret_cast<const uint4 *>(y + (size_t)best * H)[c]);
+                acc.add(bf2f(w[(size_t)t * k + bs]), reinterpret_cast<const uint4 *>(y + (size_t)best * H)[c]);
             }
         } else {
             for (int s = 0; s < k; ++s) {
                 const int r = row_of[(size_t)t * k + s];
-                add(bf2f(w[(size_t)t * k + s]), reinterpret_cast<const uint4 *>(y + (size_t)r * H)[c]);
+                acc.add(bf2f(w[(size_t)t * k + s]), reinterpret_cast<const uint4 *>(y + (size_t)r * H)[c]);
             }
         }
-        if (ORDERED && add_in) {
-            const uint4 v = reinterpret_cast<const uint4 *>(add_in + (size_t)t * H)[c];
-            const float av[8] = {lo_bf(v.x), hi_bf(v.x), lo_bf(v.y), hi_bf(v.y),
-                                 lo_bf(v.z), hi_bf(v.z), lo_bf(v.w), hi_bf(v.w)};
-#pragma unroll
-            for (int q = 0; q < 8; ++q) acc[q] = bf16_round(acc[q] + av[q]);
-        }
-        uint4 o;
-        o.x = f2bf(acc[0]) | (f2bf(acc[1]) << 16);
-        o.y = f2bf(acc[2]) | (f2bf(acc[3]) << 16);
-        o.z = f2bf(acc[4]) | (f2bf(acc[5]) << 16);
-        o.w = f2bf(acc[6]) | (f2bf(acc[7]) << 16);
-        reinterpret_cast<uint4 *>(out + (size_t)t * H)[c] = o;
+        if (ORDERED && add_in) acc.add_last(reinterpret_cast<const uint4 *>(add_in + (size_t)t * H)[c]);
+        reinterpret_cast<uint4 *>(out + (size_t)t * H)[c] = acc.result();
     }
 }
 
@@ -158,20 +187,20 @@ static int launch_merge(const void *y, const int32_t *row_of, const void *w, int
                         const void *add_in, void *out, void *stream) {
     if (!y || !row_of || !w || !out) return fail(kEInval, "merge: null pointer");
     if (T < 1 || k < 1 || H < 8 || H % 8) return fail(kEInval, "merge: need T,k >= 1 and H % 8 == 0");
-    const int64_t total = (int64_t)T * (H / 8);
-    const int blocks = (int)std::min<int64_t>((total + 255) / 256, 65536);
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     const uint16_t *yy = (const uint16_t *)y, *ww = (const uint16_t *)w, *aa = (const uint16_t *)add_in;
-    // few tokens: latency-bound, all of a thread's rows in flight at once
-    // (T=512: 7.7 us against 9.5 us); many tokens: bandwidth-bound, where the
-    // slot-at-a-time loop keeps more threads resident (T=4096: 29.5 us
-    // against 33.3 us)
-    if (k <= 8 && T <= 1024)
-        merge_kernel<8, ORDERED><<<blocks, 256, 0, s>>>(yy, row_of, ww, T, k, H, aa, (uint16_t *)out);
-    else if (k <= 16 && T <= 1024)
-        merge_kernel<16, ORDERED><<<blocks, 256, 0, s>>>(yy, row_of, ww, T, k, H, aa, (uint16_t *)out);
-    else
-        merge_kernel<0, ORDERED><<<blocks, 256, 0, s>>>(yy, row_of, ww, T, k, H, aa, (uint16_t *)out);
+    if (k <= 16) {
+        const int64_t waves = (int64_t)T * ((H / 8 + 63) / 64);
+        const int blocks = (int)std::min<int64_t>((waves + 3) / 4, 65536);
+        if (k <= 8)
+            merge_kernel<8, ORDERED><<<blocks, 256, 0, s>>>(yy, row_of, ww, T, k, H, aa, (uint16_t *)out);
+        else
+            merge_kernel<16, ORDERED><<<blocks, 256, 0, s>>>(yy, row_of, ww, T, k, H, aa, (uint16_t *)out);
+    } else {
+        const int64_t total = (int64_t)T * (H / 8);
+        const int blocks = (int)std::min<int64_t>((total + 255) / 256, 65536);
+        merge_any_kernel<ORDERED><<<blocks, 256, 0, s>>>(yy, row_of, ww, T, k, H, aa, (uint16_t *)out);
+    }
     return check_launch("merge_kernel");
 }
 

@@ -546,6 +546,31 @@ def test_merge_ordered_matches_oracle_bit_exact(orc, pd, T, k):
         assert np.array_equal(u16(out), orc.merge_ordered(y, row_of, w, add_in=add_in))
 
 
+@pytest.mark.parametrize("H", [8, 504, 520, 1536])
+@pytest.mark.parametrize("T,k", [(1, 1), (5, 9), (1025, 16), (3, 17)])
+def test_merge_row_groups_match_oracle(orc, pd, T, k, H):
+    """Row widths around the 512 columns a wave covers and k on both sides of
+    the kernels' limits (8, 16): the ordered merge bit-exact with the oracle,
+    the fp32 one within two bf16 roundings of it (its sum is fp32 in slot
+    order; the oracle's host sum may round an intermediate differently)."""
+    ops, _, _ = pd
+    rng = np.random.default_rng(29 + T + k + H)
+    y = orc.f32_to_bf16(rng.standard_normal((T * k, H)).astype(np.float32) * 0.3)
+    w = orc.f32_to_bf16(rng.random((T, k)).astype(np.float32) / k)
+    row_of = rng.permutation(T * k).astype(np.int32)
+    add = orc.f32_to_bf16(rng.standard_normal((T, H)).astype(np.float32))
+    out = torch.empty((T, H), dtype=torch.bfloat16, device=DEV)
+    for add_in in (None, add):
+        dev_add = None if add_in is None else from_u16(add_in)
+        ops.merge(from_u16(y), torch.from_numpy(row_of).to(DEV), from_u16(w), out, add_in=dev_add, mode="reference")
+        torch.cuda.synchronize()
+        assert np.array_equal(u16(out), orc.merge_ordered(y, row_of, w, add_in=add_in))
+        ops.merge(from_u16(y), torch.from_numpy(row_of).to(DEV), from_u16(w), out, add_in=dev_add)
+        torch.cuda.synchronize()
+        ref = orc.bf16_to_f32(orc.merge(y, row_of, w, add_in=add_in))
+        np.testing.assert_allclose(orc.bf16_to_f32(u16(out)), ref, rtol=2.0 ** -7, atol=1e-5)
+
+
 def test_stage_merge_matches_bf16_index_add(pd):
     ops, _, _ = pd
     rows, H = 8, 2048
