@@ -62,6 +62,17 @@ int pdscope_route_topk(const void *x, const void *gate, const float *bias, int T
                        float *probs, void *workspace, void *stream);
 
 /*
+ * pdscope_route_topk for T <= 8 tokens whose launch also computes the gate/up
+ * half of always-on shared experts, h_shared[t,i] = bf16(bf16(silu(bf16(g))) *
+ * bf16(u)) of the block shared_slot[0] (gate|up|down of intermediate shared_I;
+ * device table of one entry), h_shared [T, shared_I] bf16.
+ */
+int pdscope_route_topk_shared(const void *x, const void *gate, const float *bias, int T, int H, int E,
+                              int k, int normalize, void *logits, int32_t *ids, void *weights,
+                              float *probs, void *workspace, const void *const *shared_slot, int shared_I,
+                              void *h_shared, void *stream);
+
+/*
  * A2 gate-fallback predictor histogram: replaces the Counter over
  * route(x, next_gate).selected (expertbench/pdscope_runtime.py:245-249).
  * hist[e] = number of (t, slot) with ids[t,slot] == e; hist is overwritten.
@@ -235,6 +246,19 @@ int pdscope_merge_ordered(const void *y, const int32_t *row_of, const void *w, i
 int pdscope_swiglu_decode(const void *x, const int32_t *ids, const void *w, int k,
                           const void *const *slots, int H, int I, void *h_ws, void *out,
                           int merge_mode, void *stream);
+
+/*
+ * pdscope_swiglu_decode plus the down half of always-on shared experts over
+ * h_shared [shared_I] (pdscope_route_topk_shared): y_shared [H] bf16 is
+ * written and added unweighted to out (before the weighted sum in
+ * merge_mode 0, after it in merge_mode 1, as pdscope_merge's add_in).
+ * pdscope_decode_shared_supported: whether both calls take one token of a shape.
+ */
+int pdscope_swiglu_decode_shared(const void *x, const int32_t *ids, const void *w, int k,
+                                 const void *const *slots, int H, int I, void *h_ws,
+                                 const void *const *shared_slot, int shared_I, const void *h_shared,
+                                 void *y_shared, void *out, int merge_mode, void *stream);
+int pdscope_decode_shared_supported(int H, int I, int E, int k, int shared_I);
 
 /*
  * A1+A4+A8 for one decode token in ONE launch: replaces route

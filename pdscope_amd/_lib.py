@@ -22,6 +22,8 @@ SIGNATURES = {
     "pdscope_route_workspace_bytes": ([], _sz),
     "pdscope_route_workspace_size": ([_i32, _i32, _i32], _sz),
     "pdscope_route_topk": ([_vp, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _vp, _vp, _vp, _vp, _vp, _vp], _i32),
+    "pdscope_route_topk_shared": ([_vp, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _vp, _vp, _vp, _vp, _vp, _vp, _i32,
+                                   _vp, _vp], _i32),
     "pdscope_route_hist": ([_vp, _i32, _i32, _vp, _vp], _i32),
     "pdscope_pack": ([_vp, _i32, _i32, _i32, _vp, _vp, _vp, _vp, _vp, _vp, _vp], _i32),
     "pdscope_pack_workspace_size": ([_i32, _i32, _i32], _sz),
@@ -40,6 +42,9 @@ SIGNATURES = {
     "pdscope_merge": ([_vp, _vp, _vp, _i32, _i32, _i32, _vp, _vp, _vp], _i32),
     "pdscope_merge_ordered": ([_vp, _vp, _vp, _i32, _i32, _i32, _vp, _vp, _vp], _i32),
     "pdscope_swiglu_decode": ([_vp, _vp, _vp, _i32, _vp, _i32, _i32, _vp, _vp, _i32, _vp], _i32),
+    "pdscope_swiglu_decode_shared": ([_vp, _vp, _vp, _i32, _vp, _i32, _i32, _vp, _vp, _i32, _vp, _vp, _vp, _i32,
+                                      _vp], _i32),
+    "pdscope_decode_shared_supported": ([_i32, _i32, _i32, _i32, _i32], _i32),
     "pdscope_decode_workspace_bytes": ([], _sz),
     "pdscope_decode_layer_supported": ([_i32, _i32, _i32, _i32], _i32),
     "pdscope_decode_layer_chained_supported": ([_i32, _i32, _i32, _i32, _i32], _i32),

@@ -17,8 +17,10 @@
 //   adds them in ascending expert id in bf16 arithmetic (merge_mode 1, the
 //   reference's merge, expertbench/pdscope_runtime.py:466-468:
 //   acc = bf16(acc + bf16(w_s * y_s[j]))).  h (k*I bf16) is staged in LDS
-//   once per block.
+//   once per block.  Always-on shared experts are a further row per output
+//   column; their gate/up half runs beside the router (route.hip).
 #include "common.h"
+#include "topk.h"
 
 namespace pd {
 
@@ -77,16 +79,120 @@ __global__ __launch_bounds__(256) void decode_gateup_kernel(const uint16_t *__re
     }
 }
 
-// CPL = 16-byte chunks per lane per expert row (ceil(I / 8 / 32))
-template <int CPL>
+// Down half of always-on shared experts in the same launch (slot == nullptr: none).
+struct SharedDown {
+    const uint16_t *const *slot;  // [1] gate|up|down block
+    int I;
+    const uint16_t *h;            // [I]
+    uint16_t *y;                  // [H]
+};
+
+// CPL = 16-byte chunks per lane per expert row (ceil(I / 8 / 32)); KP slot
+// pairs (k <= 2 KP) and CS 16-byte chunks per lane of a shared row (0: none).
+// Every row of the wave's output column is loaded before h is staged, so the
+// launch, bound by the bytes of the down rows, pays one memory latency instead
+// of one per slot pair (two waves a SIMD cannot hide it).
+template <int CPL, int KP, int CS>
 __global__ __launch_bounds__(256) void decode_down_kernel(const uint16_t *__restrict__ h_ws,
                                                           const int32_t *__restrict__ ids,
                                                           const uint16_t *__restrict__ w,
                                                           const uint16_t *const *__restrict__ slots, int H,
-                                                          int I, int k, int merge_mode,
+                                                          int I, int k, int merge_mode, SharedDown sd,
                                                           uint16_t *__restrict__ out) {
+    extern __shared__ uint4 s_h[];         // k * I, then sd.I bf16
+    __shared__ float s_ys[4][2 * KP];      // per wave: bf16 y of each slot
+    const int CI = I >> 3, CSI = CS ? sd.I >> 3 : 0;
+    const int lane = lane_id(), half = lane >> 5, hl = lane & 31, wave = threadIdx.x >> 6;
+    const int j = blockIdx.x * 4 + wave;
+    const int jc = min(j, H - 1);
+    const size_t IH2 = 2 * (size_t)I * H;
+    uint4 wv[KP][CPL];
+    bool has[KP];
+#pragma unroll
+    for (int p = 0; p < KP; ++p) {
+        const int s = 2 * p + half;
+        const uint16_t *base = s < k ? slots[ids[s]] : nullptr;
+        has[p] = base != nullptr;
+        // no slot or no ready copy: read h itself (k*I elements, in bounds) and add 0
+        const uint4 *row = base ? reinterpret_cast<const uint4 *>(base + IH2 + (size_t)jc * I)
+                                : reinterpret_cast<const uint4 *>(h_ws);
+#pragma unroll
+        for (int c = 0; c < CPL; ++c) wv[p][c] = ld_nt(row + min(hl + 32 * c, CI - 1));
+    }
+    // lane s: slot s's expert id and weight, in ascending expert id for merge_mode 1
+    int order = lane, wb = 0;
+    if (lane < k) wb = w[lane];
+    if (merge_mode) {
+        const int e = lane < k ? ids[lane] : 0;
+        int rank = 0;
+        for (int s = 0; s < k; ++s) rank += __builtin_amdgcn_readlane(e, s) < e;
+        const int dst = (lane < k ? rank : lane) * 4;
+        order = __builtin_amdgcn_ds_permute(dst, lane);
+        wb = __builtin_amdgcn_ds_permute(dst, wb);
+    }
+    uint4 sv[CS ? CS : 1];
+    bool shas = false;
+    if constexpr (CS > 0) {
+        const uint16_t *base = sd.slot[0];
+        shas = base != nullptr;
+        const uint4 *row = base ? reinterpret_cast<const uint4 *>(base + 2 * (size_t)sd.I * H + (size_t)jc * sd.I)
+                                : reinterpret_cast<const uint4 *>(sd.h);
+#pragma unroll
+        for (int c = 0; c < CS; ++c) sv[c] = ld_nt(row + min(lane + 64 * c, CSI - 1));
+    }
+    for (int idx = threadIdx.x; idx < k * CI; idx += blockDim.x)
+        s_h[idx] = reinterpret_cast<const uint4 *>(h_ws)[idx];
+    for (int idx = threadIdx.x; idx < CSI; idx += blockDim.x)
+        s_h[k * CI + idx] = reinterpret_cast<const uint4 *>(sd.h)[idx];
+    __syncthreads();
+#pragma unroll
+    for (int p = 0; p < KP; ++p) {
+        const int s = min(2 * p + half, k - 1);
+        float acc = 0.0f;
+#pragma unroll
+        for (int c = 0; c < CPL; ++c) {
+            const int ch = hl + 32 * c;
+            if (ch < CI) acc = dot8(wv[p][c], s_h[s * CI + ch], acc);
+        }
+        acc = half_sum_dpp(has[p] ? acc : 0.0f);  // lanes 31 / 63 hold the sums of the two halves
+        if (hl == 31 && 2 * p + half < k) s_ys[wave][2 * p + half] = bf16_round(acc);
+    }
+    float add = 0.0f;
+    if constexpr (CS > 0) {
+        float acc = 0.0f;
+#pragma unroll
+        for (int c = 0; c < CS; ++c) {
+            const int ch = lane + 64 * c;
+            if (ch < CSI) acc = dot8(sv[c], s_h[k * CI + ch], acc);
+        }
+        add = bf16_round(wave_sum_dpp(shas ? acc : 0.0f));
+    }
+    wave_lds_sync();
+    // the weighted sum in either merge arithmetic; the shared experts' y is
+    // unweighted: first in the fp32 sum, last in the bf16 sequence
+    float total = merge_mode ? 0.0f : add;
+    for (int s = 0; s < k; ++s) {
+        const float ws = bf2f((uint32_t)__builtin_amdgcn_readlane(wb, s));
+        const float ys = s_ys[wave][__builtin_amdgcn_readlane(order, s)];
+        total = merge_mode ? bf16_round(total + bf16_round(ws * ys)) : __builtin_fmaf(ws, ys, total);
+    }
+    if (CS > 0 && merge_mode) total = bf16_round(total + add);
+    if (lane == 0 && j < H) {
+        if constexpr (CS > 0) sd.y[j] = (uint16_t)f2bf(add);
+        out[j] = (uint16_t)f2bf(total);
+    }
+}
+
+// any shape the entry point takes: one slot pair at a time
+template <int CPL>
+__global__ __launch_bounds__(256) void decode_down_any_kernel(const uint16_t *__restrict__ h_ws,
+                                                              const int32_t *__restrict__ ids,
+                                                              const uint16_t *__restrict__ w,
+                                                              const uint16_t *const *__restrict__ slots, int H,
+                                                              int I, int k, int merge_mode,
+                                                              uint16_t *__restrict__ out) {
     extern __shared__ uint4 s_h[];
-    __shared__ float s_ys[4][16];  // per wave: bf16 y of each slot (merge_mode 1)
+    __shared__ float s_ys[4][16];  // per wave: bf16 y of each slot
     const int CI = I >> 3;
     for (int idx = threadIdx.x; idx < k * CI; idx += blockDim.x)
         s_h[idx] = reinterpret_cast<const uint4 *>(h_ws)[idx];
@@ -148,15 +254,20 @@ __global__ __launch_bounds__(256) void decode_down_kernel(const uint16_t *__rest
 
 using namespace pd;
 
-PD_API int pdscope_swiglu_decode(const void *x, const int32_t *ids, const void *w, int k,
-                                 const void *const *slots, int H, int I, void *h_ws, void *out,
-                                 int merge_mode, void *stream) {
+// Slot pairs, chunks per half-wave lane and shared chunks per lane that
+// decode_down_kernel is built for; false: decode_down_any_kernel (no shared).
+static bool down_fits(int k, int I, int shared_I) {
+    return k <= 8 && I <= 6 * 256 && shared_I <= 6 * 512;
+}
+
+static int launch_decode(const void *x, const int32_t *ids, const void *w, int k, const void *const *slots, int H,
+                         int I, void *h_ws, void *out, int merge_mode, SharedDown sd, void *stream) {
     if (!x || !ids || !w || !slots || !h_ws || !out) return fail(kEInval, "decode: null pointer");
     if (merge_mode != 0 && merge_mode != 1) return fail(kEInval, "decode: merge_mode must be 0 or 1");
     if (k < 1 || k > 16) return fail(kEInval, "decode: need 1 <= k <= 16");
     if (H < 8 || H % 8 || H > 4096) return fail(kEInval, "decode: need H % 8 == 0 and H <= 4096");
     if (I < 8 || I % 8 || I > 8192) return fail(kEInval, "decode: need I % 8 == 0 and I <= 8192");
-    if ((size_t)k * I * 2 > 64 * 1024) return fail(kEInval, "decode: k*I*2 must fit 64 KiB of LDS");
+    if (((size_t)k * I + sd.I) * 2 > 64 * 1024) return fail(kEInval, "decode: k*I*2 must fit 64 KiB of LDS");
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     const uint16_t *xp = (const uint16_t *)x;
     const uint16_t *const *sp = (const uint16_t *const *)slots;
@@ -175,23 +286,63 @@ PD_API int pdscope_swiglu_decode(const void *x, const int32_t *ids, const void *
     int rc = check_launch("decode_gateup_kernel");
     if (rc) return rc;
     const int cpl = ((I >> 3) + 31) / 32;
-    const size_t lds = (size_t)k * I * 2;
+    const size_t lds = ((size_t)k * I + sd.I) * 2;
     const int dblocks = (H + 3) / 4;
+    const uint16_t *hp = (const uint16_t *)h_ws, *wp = (const uint16_t *)w;
+    if (down_fits(k, I, sd.I)) {
+        const int kp = k <= 4 ? 2 : k <= 6 ? 3 : 4, cs = sd.slot ? (sd.I <= 3 * 512 ? 3 : 6) : 0;
+        const int cc = cpl <= 3 ? 3 : 6;
+#define PD_DN(C, P, S)                                                                                          \
+    if (cc == C && kp == P && cs == S)                                                                          \
+        decode_down_kernel<C, P, S><<<dblocks, 256, lds, s>>>(hp, ids, wp, sp, H, I, k, merge_mode, sd, (uint16_t *)out);
+#define PD_DNS(C, P) PD_DN(C, P, 0) PD_DN(C, P, 3) PD_DN(C, P, 6)
+        PD_DNS(3, 2) PD_DNS(3, 3) PD_DNS(3, 4) PD_DNS(6, 2) PD_DNS(6, 3) PD_DNS(6, 4)
+#undef PD_DNS
+#undef PD_DN
+        return check_launch("decode_down_kernel");
+    }
+    if (sd.slot) return fail(kEInval, "decode: shared experts need k <= 8, I <= 1536 and a shared I <= 3072");
     switch (cpl) {
 #define PD_DN(C)                                                                                           \
     case C:                                                                                                \
-        decode_down_kernel<C><<<dblocks, 256, lds, s>>>((const uint16_t *)h_ws, ids, (const uint16_t *)w, sp, H, \
-                                                        I, k, merge_mode, (uint16_t *)out);                \
+        decode_down_any_kernel<C><<<dblocks, 256, lds, s>>>(hp, ids, wp, sp, H, I, k, merge_mode, (uint16_t *)out); \
         break;
         PD_DN(1) PD_DN(2) PD_DN(3) PD_DN(4) PD_DN(5) PD_DN(6) PD_DN(7) PD_DN(8)
 #undef PD_DN
     default:
         if (cpl <= 32) {
-            decode_down_kernel<32><<<dblocks, 256, lds, s>>>((const uint16_t *)h_ws, ids, (const uint16_t *)w, sp,
-                                                             H, I, k, merge_mode, (uint16_t *)out);
+            decode_down_any_kernel<32><<<dblocks, 256, lds, s>>>(hp, ids, wp, sp, H, I, k, merge_mode,
+                                                                 (uint16_t *)out);
         } else {
             return fail(kEInval, "decode: unsupported I");
         }
     }
     return check_launch("decode_down_kernel");
+}
+
+PD_API int pdscope_swiglu_decode(const void *x, const int32_t *ids, const void *w, int k,
+                                 const void *const *slots, int H, int I, void *h_ws, void *out,
+                                 int merge_mode, void *stream) {
+    return launch_decode(x, ids, w, k, slots, H, I, h_ws, out, merge_mode, SharedDown{nullptr, 0, nullptr, nullptr},
+                         stream);
+}
+
+PD_API int pdscope_swiglu_decode_shared(const void *x, const int32_t *ids, const void *w, int k,
+                                        const void *const *slots, int H, int I, void *h_ws,
+                                        const void *const *shared_slot, int shared_I, const void *h_shared,
+                                        void *y_shared, void *out, int merge_mode, void *stream) {
+    if (!shared_slot || !h_shared || !y_shared || shared_I < 8 || shared_I % 8)
+        return fail(kEInval, "decode_shared: bad shared arguments");
+    return launch_decode(x, ids, w, k, slots, H, I, h_ws, out, merge_mode,
+                         SharedDown{(const uint16_t *const *)shared_slot, shared_I, (const uint16_t *)h_shared,
+                                    (uint16_t *)y_shared},
+                         stream);
+}
+
+// Whether pdscope_route_topk_shared + pdscope_swiglu_decode_shared run one
+// token of this shape.
+PD_API int pdscope_decode_shared_supported(int H, int I, int E, int k, int shared_I) {
+    return H >= 16 && H % 16 == 0 && H <= 4096 && I >= 8 && I % 8 == 0 && E >= 32 && E <= 256 && E % 32 == 0 &&
+           k >= 1 && k <= E && shared_I >= 8 && shared_I % 8 == 0 && down_fits(k, I, shared_I) &&
+           ((size_t)k * I + shared_I) * 2 <= 64 * 1024;
 }

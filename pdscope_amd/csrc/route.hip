@@ -35,16 +35,77 @@ constexpr int kGemvMaxT = 8;
 // router row once and dots it with the <= 8 token rows.  The last block to
 // finish (device-scope counter in the workspace, reset by that block) runs
 // the softmax/top-k for every token.
+//
+// SHARED: the launch has further blocks, which compute the gate/up half of
+// always-on shared experts (h = bf16(bf16(silu(bf16(g))) * bf16(u)), two rows
+// per wave as decode_gateup_kernel).  They need only the tokens, so their
+// weights stream while the router's blocks and its one routing block, bound by
+// latency, leave the memory idle.
+struct SharedGateUp {
+    const uint16_t *const *slot;  // [1] gate|up|down block
+    int I;
+    uint16_t *h;                  // [T, I]
+};
+
 template <int NCH>
+__device__ __forceinline__ void shared_gateup_rows(const SharedGateUp &sg, const uint16_t *__restrict__ x, int T,
+                                                   int H, int q0) {
+    const int lane = lane_id();
+    if (q0 >= sg.I) return;
+    const int C = H >> 3;
+    const uint16_t *base = sg.slot[0];
+    uint4 gv[2][NCH], uv[2][NCH];
+#pragma unroll
+    for (int it = 0; it < 2; ++it) {
+        const int q = min(q0 + it, sg.I - 1);
+        // no copy: read the activation row (H elements, in bounds) and store h = 0
+        const uint16_t *grow = base ? base + (size_t)q * H : x;
+        const uint16_t *urow = base ? base + (size_t)(sg.I + q) * H : x;
+#pragma unroll
+        for (int j = 0; j < NCH; ++j) {
+            gv[it][j] = ld_nt(grow + 8 * min(lane + 64 * j, C - 1));
+            uv[it][j] = ld_nt(urow + 8 * min(lane + 64 * j, C - 1));
+        }
+    }
+    for (int t = 0; t < T; ++t) {
+        const uint4 *xrow = reinterpret_cast<const uint4 *>(x + (size_t)t * H);
+        uint4 xv[NCH];
+#pragma unroll
+        for (int j = 0; j < NCH; ++j) xv[j] = xrow[min(lane + 64 * j, C - 1)];
+#pragma unroll
+        for (int it = 0; it < 2; ++it) {
+            float g = 0.0f, u = 0.0f;
+#pragma unroll
+            for (int j = 0; j < NCH; ++j)
+                if (lane + 64 * j < C) {
+                    g = dot8(gv[it][j], xv[j], g);
+                    u = dot8(uv[it][j], xv[j], u);
+                }
+            g = wave_sum_dpp(g);
+            u = wave_sum_dpp(u);
+            if (lane == 0 && q0 + it < sg.I) {
+                const float a = bf16_round(silu_f32(bf16_round(g)));
+                sg.h[(size_t)t * sg.I + q0 + it] = base ? (uint16_t)f2bf(a * bf16_round(u)) : (uint16_t)0;
+            }
+        }
+    }
+}
+
+template <int NCH, bool SHARED>
 __global__ __launch_bounds__(256) void route_gemv_kernel(
     const uint16_t *__restrict__ x, const uint16_t *__restrict__ gate, const float *__restrict__ bias,
     int T, int H, int E, int k, int normalize, uint16_t *__restrict__ logits,
     int32_t *__restrict__ ids, uint16_t *__restrict__ weights, float *__restrict__ probs,
-    uint32_t *__restrict__ counter) {
+    uint32_t *__restrict__ counter, SharedGateUp sg) {
     __shared__ float s_logit[kGemvMaxT * 256];
     __shared__ TopkScratch s_tk[4];
     __shared__ int s_last;
     const int lane = lane_id();
+    const int nroute = (E + 3) / 4;
+    if (SHARED && (int)blockIdx.x >= nroute) {
+        shared_gateup_rows<NCH>(sg, x, T, H, (((int)blockIdx.x - nroute) * 4 + (int)(threadIdx.x >> 6)) * 2);
+        return;
+    }
     const int e = blockIdx.x * 4 + (threadIdx.x >> 6);
     const int C = H >> 3;  // 16-byte chunks per row; lane owns chunks lane + 64*j
     if (e < E) {
@@ -69,7 +130,7 @@ __global__ __launch_bounds__(256) void route_gemv_kernel(
     __syncthreads();
     if (threadIdx.x == 0) {
         uint32_t prev = atomicAdd(counter, 1u);
-        s_last = (prev == gridDim.x - 1);
+        s_last = (prev == (uint32_t)nroute - 1);
     }
     __syncthreads();
     if (!s_last) return;
@@ -272,31 +333,61 @@ PD_API size_t pdscope_route_workspace_size(int T, int H, int E) {
     return 256 + (size_t)(H / kc) * (size_t)T * (size_t)E * sizeof(float);
 }
 
-PD_API int pdscope_route_topk(const void *x, const void *gate, const float *bias, int T, int H, int E,
-                              int k, int normalize, void *logits, int32_t *ids, void *weights,
-                              float *probs, void *workspace, void *stream) {
+// Checks shared by the router entry points.
+static int route_check(const void *x, const void *gate, int T, int H, int E, int k, const void *logits,
+                       const void *ids, const void *weights, const void *workspace) {
     if (!x || !gate || !logits || !ids || !weights) return fail(kEInval, "route: null tensor pointer");
     if (T < 1 || H < 16 || H % 16) return fail(kEInval, "route: need T >= 1 and H % 16 == 0");
     if (E < 32 || E > 256 || E % 32) return fail(kEInval, "route: need E % 32 == 0 and E <= 256");
     if (k < 1 || k > 16 || k > E) return fail(kEInval, "route: need 1 <= k <= min(E, 16)");
     if (!workspace) return fail(kEInval, "route: workspace (pdscope_route_workspace_size bytes) is required");
-    hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-    if (T <= kGemvMaxT) {
-        const int nch = (H / 8 + 63) / 64;
-        switch (nch) {
-#define PD_RG(N)                                                                                           \
-    case N:                                                                                                \
-        route_gemv_kernel<N><<<(E + 3) / 4, 256, 0, s>>>((const uint16_t *)x, (const uint16_t *)gate, bias, T, H, E, k, \
-                                                         normalize, (uint16_t *)logits, ids, (uint16_t *)weights,  \
-                                                         probs, (uint32_t *)workspace);                    \
-        break;
-            PD_RG(1) PD_RG(2) PD_RG(3) PD_RG(4) PD_RG(5) PD_RG(6) PD_RG(7) PD_RG(8)
-#undef PD_RG
-        default:
-            return fail(kEInval, "route: small-T path needs H <= 4096");
-        }
-        return check_launch("route_gemv_kernel");
+    return kOk;
+}
+
+// The small-T launch; with sg.slot, its extra blocks compute the shared gate/up half.
+static int launch_route_gemv(const void *x, const void *gate, const float *bias, int T, int H, int E, int k,
+                             int normalize, void *logits, int32_t *ids, void *weights, float *probs,
+                             void *workspace, SharedGateUp sg, hipStream_t s) {
+    const int nroute = (E + 3) / 4;
+    const int blocks = nroute + (sg.slot ? (sg.I + 7) / 8 : 0);
+    switch ((H / 8 + 63) / 64) {
+#define PD_RG(N)                                                                                                  \
+    case N: {                                                                                                     \
+        auto fn = sg.slot ? route_gemv_kernel<N, true> : route_gemv_kernel<N, false>;                             \
+        fn<<<blocks, 256, 0, s>>>((const uint16_t *)x, (const uint16_t *)gate, bias, T, H, E, k, normalize,       \
+                                  (uint16_t *)logits, ids, (uint16_t *)weights, probs, (uint32_t *)workspace, sg); \
+        break;                                                                                                    \
     }
+        PD_RG(1) PD_RG(2) PD_RG(3) PD_RG(4) PD_RG(5) PD_RG(6) PD_RG(7) PD_RG(8)
+#undef PD_RG
+    default:
+        return fail(kEInval, "route: small-T path needs H <= 4096");
+    }
+    return check_launch("route_gemv_kernel");
+}
+
+PD_API int pdscope_route_topk_shared(const void *x, const void *gate, const float *bias, int T, int H, int E, int k,
+                                     int normalize, void *logits, int32_t *ids, void *weights, float *probs,
+                                     void *workspace, const void *const *shared_slot, int shared_I, void *h_shared,
+                                     void *stream) {
+    const int rc = route_check(x, gate, T, H, E, k, logits, ids, weights, workspace);
+    if (rc != kOk) return rc;
+    if (T > kGemvMaxT) return fail(kEInval, "route_topk_shared: needs T <= 8");
+    if (!shared_slot || !h_shared || shared_I < 1) return fail(kEInval, "route_topk_shared: bad shared arguments");
+    return launch_route_gemv(x, gate, bias, T, H, E, k, normalize, logits, ids, weights, probs, workspace,
+                             SharedGateUp{(const uint16_t *const *)shared_slot, shared_I, (uint16_t *)h_shared},
+                             reinterpret_cast<hipStream_t>(stream));
+}
+
+PD_API int pdscope_route_topk(const void *x, const void *gate, const float *bias, int T, int H, int E,
+                              int k, int normalize, void *logits, int32_t *ids, void *weights,
+                              float *probs, void *workspace, void *stream) {
+    int rc = route_check(x, gate, T, H, E, k, logits, ids, weights, workspace);
+    if (rc != kOk) return rc;
+    hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+    if (T <= kGemvMaxT)
+        return launch_route_gemv(x, gate, bias, T, H, E, k, normalize, logits, ids, weights, probs, workspace,
+                                 SharedGateUp{nullptr, 0, nullptr}, s);
     const int kc = route_kchunk(H);
     const int KS = H / kc;
     float *part = reinterpret_cast<float *>(static_cast<char *>(workspace) + 256);
@@ -320,7 +411,7 @@ PD_API int pdscope_route_topk(const void *x, const void *gate, const float *bias
         return fail(kEInval, "route: unsupported K chunk");
     }
     }
-    int rc = check_launch(staged ? "route_partial_lds_kernel" : "route_partial_kernel");
+    rc = check_launch(staged ? "route_partial_lds_kernel" : "route_partial_kernel");
     if (rc) return rc;
     const int g2 = (T + 3) / 4;
     if (E <= 64)

@@ -1,7 +1,8 @@
 """One MoE layer on the gfx950 kernels with a preallocated workspace.
 
 ``moe_forward`` is the whole GPU layer for experts addressed through a slot
-table: route (K1) -> decode GEMV (K4) for T == 1, or pack (K2) -> balanced tile
+table: route (K1) -> decode GEMV (K4) for T == 1 (with or without shared
+experts), or pack (K2) -> balanced tile
 schedule -> grouped SwiGLU (K3) -> merge (K5) for T > 1.  Nothing is
 allocated and nothing is read back to the host, so the call can be captured
 in a hipGraph (torch.cuda.CUDAGraph) and replayed.
@@ -95,6 +96,16 @@ def route(x, gate, ws: MoEWorkspace, *, normalize=True, bias=None):
 
 # column width of the gate|up tile for each row-tile height of the grouped kernel
 _GATEUP_COLS = {32: 128, 64: 128, 128: 128, 256: 128, 384: 64}
+
+
+def decode_shared_fits(ws: MoEWorkspace) -> bool:
+    """Whether one token with shared experts runs on the streaming GEMV
+    kernels (three launches, no side stream) instead of the grouped ones
+    (seven launches on two streams, whose 32-row tiles hold one row:
+    DeepSeek-V2-Lite shape, 82 us a layer against 39).  Only shapes that the
+    grouped kernels take as well."""
+    return (ws.H % 256 == 0 and ws.I % 128 == 0 and ws.shared_I % 64 == 0
+            and ops.decode_shared_supported(ws.H, ws.I, ws.E, ws.k, ws.shared_I))
 
 
 def shared_block_m(T: int, I: int) -> int:
@@ -200,7 +211,8 @@ def moe_forward(x, gate, slots, ws: MoEWorkspace, *, normalize=True, bias=None, 
     T == 1 runs the single-launch decode kernel (K4f) when the shape and the
     device allow it (fused_decode), else route (K1) + decode GEMV (K4).
     shared_slot (int64 [1] device table) adds always-on shared experts
-    (DeepSeek-V2); the workspace must have been built with shared_I.
+    (DeepSeek-V2); the workspace must have been built with shared_I.  One token
+    then runs on the decode GEMV kernels (decode_shared_fits).
     next_gate / pred_out (T == 1 on the single-launch kernel only, see
     ops.decode_chained_supported): the next layer's gate-fallback prediction,
     top-k of next_gate . x, is written to pred_out [k] int32 by the same launch.
@@ -209,6 +221,14 @@ def moe_forward(x, gate, slots, ws: MoEWorkspace, *, normalize=True, bias=None, 
     if shared_slot is not None:
         if not ws.shared_I:
             raise ValueError("shared experts need a workspace built with shared_I")
+        if T == 1 and block_m is None and decode_shared_fits(ws):
+            logits, ids, weights, _ = ws.views(1)
+            out = ws.out[:1]
+            ops.decode_shared_layer(x, gate, slots, ws.I, ws.k, normalize, shared_slot, ws.shared_I, bias=bias,
+                                    out=out, logits=logits, ids=ids, weights=weights, h_ws=ws.h_ws,
+                                    h_shared=ws.h_shared, y_shared=ws.y_shared[:1], workspace=ws.route_ws,
+                                    merge=merge)
+            return out, logits, ids, weights
         # the shared experts need only x: they run on a side stream beside the
         # routing and the routed experts (a one-expert launch alone does not
         # fill the device) and join before the merge adds their output

@@ -302,6 +302,46 @@ def swiglu_decode(x, ids, w, slots, H, I, h_ws, out, *, merge="fused"):
     return out
 
 
+def decode_shared_supported(H, I, E, k, shared_I) -> bool:
+    """Whether decode_shared_layer runs one token of this shape."""
+    return bool(_lib.load().pdscope_decode_shared_supported(H, I, E, k, shared_I))
+
+
+def decode_shared_layer(x, gate, slots, I, top_k, normalize, shared_slot, shared_I, *, bias=None, out, logits, ids,
+                        weights, h_ws, h_shared, y_shared, workspace, merge="fused"):
+    """One token through a layer with always-on shared experts in three
+    launches: router + the shared gate/up half, routed gate/up, down of both +
+    merge.  y_shared [1, H] receives the shared experts' output."""
+    _need(x, "inputs", BF16, 2)
+    dev = x.device
+    _need(gate, "gate", BF16, 2, dev)
+    E, H = gate.shape
+    for t, n in ((slots, "slots"), (shared_slot, "shared_slot")):
+        _need(t, n, torch.int64, 1, dev)
+    if bias is not None:
+        _need(bias, "bias", torch.float32, 1, dev)
+        if bias.numel() != E:
+            raise ValueError("bias must have one entry per expert")
+    _need(ids, "ids", torch.int32, None, dev)
+    for t, n, size in ((x, "x", H), (out, "out", H), (logits, "logits", E), (weights, "weights", top_k),
+                       (y_shared, "y_shared", H)):
+        _need(t, n, BF16, None, dev)
+        if t.numel() != size:
+            raise ValueError(f"decode_shared_layer expects one token: {n} must hold {size} values")
+    for t, n, size in ((h_ws, "h_ws", top_k * I), (h_shared, "h_shared", shared_I)):
+        _need(t, n, BF16, None, dev)
+        if t.numel() < size:
+            raise ValueError(f"decode_shared_layer: {n} must hold {size} values")
+    if ids.numel() != top_k or slots.numel() < E or workspace.numel() < route_workspace_size(1, H, E):
+        raise ValueError("decode_shared_layer: ids must hold k, slots E entries and workspace the router's scratch")
+    mode, stream = merge_mode(merge), _stream(dev)
+    _lib.call("pdscope_route_topk_shared", _p(x), _p(gate), _p(bias), 1, H, E, top_k, int(bool(normalize)),
+              _p(logits), _p(ids), _p(weights), None, _p(workspace), _p(shared_slot), shared_I, _p(h_shared), stream)
+    _lib.call("pdscope_swiglu_decode_shared", _p(x), _p(ids), _p(weights), top_k, _p(slots), H, I, _p(h_ws),
+              _p(shared_slot), shared_I, _p(h_shared), _p(y_shared), _p(out), mode, stream)
+    return out
+
+
 _decode_ws = {}
 _decode_ok = {}
 

@@ -608,3 +608,69 @@ def test_bound_decode_equals_the_chained_launch_and_reads_back(pd):
                   ctypes.addressof(plain_words), ctypes.addressof(plain_words) + 64, ctypes.byref(handle))
     assert handle.value is None
     _assert_sync_clean(ops, H)
+
+
+# one token with always-on shared experts on the streaming GEMV kernels: slot
+# pairs 2..4 with an odd k, row chunks on both sides of their limits, the
+# shared row shorter and longer than three chunks a lane, E of one wave and four
+SHARED_SHAPES = [
+    dict(H=2048, I=1408, E=64, k=6, Is=2816, normalize=False),   # the DeepSeek-V2-Lite layer
+    dict(H=256, I=128, E=32, k=1, Is=64, normalize=True),
+    dict(H=1024, I=896, E=256, k=7, Is=1600, normalize=True),
+    dict(H=4096, I=1536, E=64, k=8, Is=3072, normalize=False),
+]
+
+
+@pytest.mark.parametrize("merge", ["fused", "reference"])
+@pytest.mark.parametrize("shape", SHARED_SHAPES, ids=lambda s: f"H{s['H']}_I{s['I']}_E{s['E']}_k{s['k']}")
+def test_one_token_with_shared_experts(orc, pd, shape, merge):
+    """moe_forward of one token with shared experts: routing bitwise the
+    router's, the shared output and the layer output within bf16 tolerance of
+    the oracle, and equal to the grouped path (block_m given) up to the order
+    of the fp32 sums (each expert value may differ by one bf16 rounding)."""
+    ops, layer, synthetic = pd
+    H, I, E, k, Is = (shape[n] for n in ("H", "I", "E", "k", "Is"))
+    lay = synthetic.make_layer(H, I, E, k, shape["normalize"], seed=H + I + k, device=DEV, shared_I=Is)
+    x = synthetic.make_tokens(1, H, seed=H + 1, device=DEV)
+    slots = ops.slot_table([lay.experts[e] for e in range(E)], DEV)
+    shared = ops.slot_table([lay.shared], DEV)
+    ws = layer.MoEWorkspace(2, H, I, E, k, DEV, shared_I=Is)
+    assert layer.decode_shared_fits(ws)
+    for bias in (None, torch.linspace(-0.5, 0.5, E, device=DEV)):
+        out, logits, ids, w = layer.moe_forward(x, lay.gate, slots, ws, normalize=shape["normalize"], bias=bias,
+                                                shared_slot=shared, merge=merge)
+        torch.cuda.synchronize()
+        rl, ri, rw, _ = ops.route_topk(x, lay.gate, k, shape["normalize"], bias=bias)
+        assert torch.equal(ids, ri) and torch.equal(w, rw) and torch.equal(logits, rl)
+        sh = u16(lay.shared)
+        n = Is * H
+        shared_ref = orc.expert_forward(u16(x), sh[:n].reshape(Is, H), sh[n:2 * n].reshape(Is, H),
+                                        sh[2 * n:].reshape(H, Is))
+        m = err_metrics(orc.bf16_to_f32(u16(ws.y_shared[:1])), orc.bf16_to_f32(shared_ref))
+        assert m["max_rel"] <= MAX_REL and m["mean_abs"] <= MEAN_ABS, m
+        got = out.clone()
+        wg = layer.MoEWorkspace(2, H, I, E, k, DEV, shared_I=Is)
+        ref, *_ = layer.moe_forward(x, lay.gate, slots, wg, normalize=shape["normalize"], bias=bias,
+                                    shared_slot=shared, merge=merge, block_m=32)
+        torch.cuda.synchronize()
+        m = err_metrics(got.float().cpu().numpy(), ref.float().cpu().numpy())
+        assert m["max_rel"] <= MAX_REL and m["mean_abs"] <= MEAN_ABS, m
+
+
+def test_one_token_with_shared_experts_without_copies(pd):
+    """A routed or shared slot without a copy (null entry) contributes zero;
+    shapes outside the kernels stay on the grouped path."""
+    ops, layer, synthetic = pd
+    H, I, E, k, Is = 512, 256, 32, 4, 256
+    lay = synthetic.make_layer(H, I, E, k, True, seed=5, device=DEV, shared_I=Is)
+    x = synthetic.make_tokens(1, H, seed=6, device=DEV)
+    slots = torch.zeros(E, dtype=torch.int64, device=DEV)
+    none = torch.zeros(1, dtype=torch.int64, device=DEV)
+    ws = layer.MoEWorkspace(1, H, I, E, k, DEV, shared_I=Is)
+    for shared in (none, ops.slot_table([lay.shared], DEV)):
+        out, _, _, _ = layer.moe_forward(x, lay.gate, slots, ws, shared_slot=shared)
+        torch.cuda.synchronize()
+        assert torch.equal(out, ws.y_shared[:1])
+        assert bool((out == 0).all()) == (shared is none)
+    assert not layer.decode_shared_fits(layer.MoEWorkspace(1, 512, 256, 32, 9, DEV, shared_I=Is))
+    assert not layer.decode_shared_fits(layer.MoEWorkspace(1, 512, 192, 32, 4, DEV, shared_I=Is))
