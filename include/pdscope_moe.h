@@ -208,6 +208,18 @@ int pdscope_swiglu_grouped_down(const void *h_ws, const int32_t *offsets, const 
                                 const void *const *slots, int H, int I, void *y, void *stream);
 
 /*
+ * The gate/up half for 384-row or 256-row tiles, chosen on the device from
+ * the two m-tile counts: tile_start_384 / tile_start_256 are the prefixes of
+ * one balanced order (pdscope_schedule_balanced_pair and
+ * pdscope_pack_schedule_balanced with block sizes 384 and 256), max_tiles_*
+ * bound their last entries.  Limits: H % 256 == 0 and I % 128 == 0.
+ */
+int pdscope_swiglu_grouped_gateup_pair(const void *x, const int32_t *perm_token, const int32_t *offsets,
+                                       const int32_t *sel, int nsel, const int32_t *tile_start_384,
+                                       int max_tiles_384, const int32_t *tile_start_256, int max_tiles_256,
+                                       const void *const *slots, int H, int I, void *h_ws, void *stream);
+
+/*
  * A8 fused weighted merge: replaces the index_add_ merge
  * (expertbench/pdscope_runtime.py:450-469).
  *   out[t,:] = bf16( add_in[t,:] + sum_s w[t,s] * y[row_of[t*k+s],:] )

@@ -15,6 +15,7 @@
 // with a 16-byte-chunk XOR swizzle applied on the source side (see Geo),
 // so fragment reads are bank-conflict free.
 // MFMA: v_mfma_f32_32x32x16_bf16, fp32 accumulation.
+#include <algorithm>
 #include <type_traits>
 
 #include "common.h"
@@ -133,9 +134,12 @@ __device__ __forceinline__ void wait_stage(int younger) {
 // XCD b % 8): all n-tiles of an m-tile share the gathered activation rows
 // in one L2, and the m-tiles of one expert read the same weight tiles at
 // the same time from one L2.
+template <int BM, int BN, int BK, int SA, int SB>
+constexpr int kRingBytes = (SA * BM + SB * BN) * BK * 2;
+
 template <int BM, int BN, int BK, int WM, int WN, int SA, int SB, bool ILV, bool GATEUP, int OCC, int FK>
-__global__ __launch_bounds__(64 * WM * WN, OCC == 1 ? 1 : OCC * WM * WN / 4) void grouped_kernel(
-    const uint16_t *__restrict__ a_src, const int32_t *__restrict__ perm_token,
+__device__ __forceinline__ void grouped_tile(
+    uint8_t *smem, const uint16_t *__restrict__ a_src, const int32_t *__restrict__ perm_token,
     const int32_t *__restrict__ offsets, const int32_t *__restrict__ sel, int nsel,
     const int32_t *__restrict__ tile_start, const uint16_t *const *__restrict__ slots, int H, int I,
     uint16_t *__restrict__ out) {
@@ -154,7 +158,7 @@ __global__ __launch_bounds__(64 * WM * WN, OCC == 1 ? 1 : OCC * WM * WN / 4) voi
     static_assert(!SPLIT || (SA - 1) * AL <= 24, "A-wave waits count live loads up to wait_vm_rt's range");
     constexpr int ASTAGE = BM * G::RB, BSTAGE = BN * G::RB;
     static_assert(OCC * (SA * ASTAGE + SB * BSTAGE) <= 160 * 1024, "LDS of OCC workgroups per CU");
-    __shared__ __attribute__((aligned(1024))) uint8_t smem[SA * ASTAGE + SB * BSTAGE];
+    static_assert(SA * ASTAGE + SB * BSTAGE == kRingBytes<BM, BN, BK, SA, SB>, "LDS ring");
     uint8_t *const ring_a = smem;
     uint8_t *const ring_b = smem + SA * ASTAGE;
 
@@ -500,6 +504,43 @@ __global__ __launch_bounds__(64 * WM * WN, OCC == 1 ? 1 : OCC * WM * WN / 4) voi
     }
 }
 
+template <int BM, int BN, int BK, int WM, int WN, int SA, int SB, bool ILV, bool GATEUP, int OCC, int FK>
+__global__ __launch_bounds__(64 * WM * WN, OCC == 1 ? 1 : OCC * WM * WN / 4) void grouped_kernel(
+    const uint16_t *__restrict__ a_src, const int32_t *__restrict__ perm_token,
+    const int32_t *__restrict__ offsets, const int32_t *__restrict__ sel, int nsel,
+    const int32_t *__restrict__ tile_start, const uint16_t *const *__restrict__ slots, int H, int I,
+    uint16_t *__restrict__ out) {
+    __shared__ __attribute__((aligned(1024))) uint8_t smem[kRingBytes<BM, BN, BK, SA, SB>];
+    grouped_tile<BM, BN, BK, WM, WN, SA, SB, ILV, GATEUP, OCC, FK>(smem, a_src, perm_token, offsets, sel, nsel,
+                                                                   tile_start, slots, H, I, out);
+}
+
+// Gate/up for a mean of about 200..320 rows per expert, where the better tile
+// depends on how the rows are spread and only the device knows that: a
+// 384-row tile (128 columns) holds most experts of a uniform routing whole,
+// where 256-row tiles (256 columns) would read the weights of every expert
+// with more than 256 rows twice; a skewed routing has experts of many tiles
+// either way, and the wider tile then reads their rows half as often.  Every
+// block compares the two m-tile counts of the same order, which the schedule
+// launch writes for both heights, and runs one body: 384 rows where they save
+// a quarter of the m-tiles or more.  Qwen shape, T=4096: uniform (128 tiles
+// against 190) 275 us on 384 rows, 280 on 256; Zipf 341 against 286.
+__global__ __launch_bounds__(512, 1) void grouped_gateup_pair_kernel(
+    const uint16_t *__restrict__ x, const int32_t *__restrict__ perm_token, const int32_t *__restrict__ offsets,
+    const int32_t *__restrict__ sel, int nsel, const int32_t *__restrict__ tile_start_384,
+    const int32_t *__restrict__ tile_start_256, const uint16_t *const *__restrict__ slots, int H, int I,
+    uint16_t *__restrict__ h_ws) {
+    constexpr int B384 = kRingBytes<384, 128, 64, 2, 4>, B256 = kRingBytes<256, 256, 64, 2, 3>;
+    __shared__ __attribute__((aligned(1024))) uint8_t smem[B384 > B256 ? B384 : B256];
+    const int m384 = tile_start_384[nsel], m256 = tile_start_256[nsel];
+    if (4 * m384 <= 3 * m256)
+        grouped_tile<384, 128, 64, 4, 2, 2, 4, true, true, 1, 32>(smem, x, perm_token, offsets, sel, nsel,
+                                                                  tile_start_384, slots, H, I, h_ws);
+    else
+        grouped_tile<256, 256, 64, 2, 4, 2, 3, true, true, 1, 16>(smem, x, perm_token, offsets, sel, nsel,
+                                                                  tile_start_256, slots, H, I, h_ws);
+}
+
 // phase: 1 = gate/up only, 2 = down only, 3 = both
 // PH: the phases (1 gate/up, 2 down) this tile configuration serves
 template <int BM, int BN, int BK, int WM, int WN, int SA, int SB, bool ILV = false, int PH = 3, int OCC = 1,
@@ -585,7 +626,10 @@ int grouped_entry(int phase, const void *x, const int32_t *perm_token, const int
         // split load roles with 2 + 3 stages fill the 160 KB of LDS
         // (T=4096, Zipf routing: gate/up 338 -> 299 us, down 199 -> 173 us;
         // uniform: down 190 -> 161 us; bit-identical)
-        return launch_grouped<256, 256, 64, 2, 4, 2, 3, false, 3, 1, 16>(phase, xp, perm_token, offsets, sel, nsel,
+        // 32-row blocks dealt to the two wave rows in turn: an expert of fewer
+        // rows than the tile keeps both busy (T=2048, 128 rows each: gate/up
+        // 163 -> 153 us, down 96 -> 90; T=4096 Zipf down 173 -> 162)
+        return launch_grouped<256, 256, 64, 2, 4, 2, 3, true, 3, 1, 16>(phase, xp, perm_token, offsets, sel, nsel,
                                                                          tile_start, max_tiles, sp, H, I,
                                                                          (uint16_t *)h_ws, (uint16_t *)y, s);
     case 384:
@@ -638,6 +682,24 @@ PD_API int pdscope_swiglu_grouped_gateup(const void *x, const int32_t *perm_toke
                                          void *stream) {
     return grouped_entry(1, x, perm_token, offsets, sel, nsel, tile_start, max_tiles, block_m, slots, H, I, h_ws,
                          nullptr, stream);
+}
+
+PD_API int pdscope_swiglu_grouped_gateup_pair(const void *x, const int32_t *perm_token, const int32_t *offsets,
+                                              const int32_t *sel, int nsel, const int32_t *tile_start_384,
+                                              int max_tiles_384, const int32_t *tile_start_256, int max_tiles_256,
+                                              const void *const *slots, int H, int I, void *h_ws, void *stream) {
+    if (!x || !perm_token || !offsets || !sel || !tile_start_384 || !tile_start_256 || !slots || !h_ws)
+        return fail(kEInval, "grouped: null pointer");
+    if (nsel < 1 || max_tiles_384 < 1 || max_tiles_256 < 1)
+        return fail(kEInval, "grouped: need nsel >= 1 and max_tiles >= 1");
+    if (H % 256 || I % 128 || H < 256 || I < 128)
+        return fail(kEInval, "grouped: the tile pair needs H % 256 == 0 and I % 128 == 0");
+    if (max_tiles_384 > (1 << 22) || max_tiles_256 > (1 << 22)) return fail(kEInval, "grouped: max_tiles too large");
+    const size_t n = std::max((size_t)max_tiles_384 * (size_t)(I / 64), (size_t)max_tiles_256 * (size_t)(I / 128));
+    grouped_gateup_pair_kernel<<<(unsigned)((n + 7) / 8 * 8), 512, 0, reinterpret_cast<hipStream_t>(stream)>>>(
+        (const uint16_t *)x, perm_token, offsets, sel, nsel, tile_start_384, tile_start_256,
+        (const uint16_t *const *)slots, H, I, (uint16_t *)h_ws);
+    return check_launch("grouped_gateup_pair_kernel");
 }
 
 PD_API int pdscope_swiglu_grouped_down(const void *h_ws, const int32_t *offsets, const int32_t *sel, int nsel,

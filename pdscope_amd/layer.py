@@ -102,7 +102,7 @@ def decode_shared_fits(ws: MoEWorkspace) -> bool:
     """Whether one token with shared experts runs on the streaming GEMV
     kernels (three launches, no side stream) instead of the grouped ones
     (seven launches on two streams, whose 32-row tiles hold one row:
-    DeepSeek-V2-Lite shape, 82 us a layer against 39).  Only shapes that the
+    DeepSeek-V2-Lite shape, 82 us a layer against 34).  Only shapes that the
     grouped kernels take as well."""
     return (ws.H % 256 == 0 and ws.I % 128 == 0 and ws.shared_I % 64 == 0
             and ops.decode_shared_supported(ws.H, ws.I, ws.E, ws.k, ws.shared_I))
@@ -169,8 +169,9 @@ def down_block_m(bm: int, H: int, I: int) -> int:
     """Row tile of the down launch for a gate/up row tile `bm`: the 384-row
     gate/up tile is 128 columns wide, and the down projection (K = I) runs
     faster on 256x256 tiles that read each h row half as often (T=4096
-    Qwen shape: 196 us against 222 us), where the shape allows them
-    (H % 256 == 0, I % 128 == 0); other tiles are shared."""
+    Qwen shape: 157 us against 164 us), where the shape allows them
+    (H % 256 == 0, I % 128 == 0); other tiles are shared.  With a second
+    row tile the gate/up launch takes either of the two, by the rows."""
     return 256 if bm == 384 and H % 256 == 0 and I % 128 == 0 else bm
 
 
@@ -196,7 +197,8 @@ def grouped_ffn(x, packed, sel, bm, max_tiles, slots, ws: MoEWorkspace, *, max_t
     tile_down = ws.tile_start_down[:nsel + 1]
     if not scheduled:
         ops.schedule(packed.counts, sel, bm, out=tile_start, order=order, block_m2=bmd, out2=tile_down)
-    ops.swiglu_grouped_gateup(x, perm, packed.offsets, order, tile_start, max_tiles, bm, slots, H, I, ws.h_ws)
+    ops.swiglu_grouped_gateup_pair(x, perm, packed.offsets, order, tile_start, max_tiles, tile_down, max_tiles_down,
+                                   slots, H, I, ws.h_ws)
     ops.swiglu_grouped_down(ws.h_ws, packed.offsets, order, tile_down, max_tiles_down, bmd, slots, H, I, ws.y)
 
 

@@ -267,6 +267,20 @@ def swiglu_grouped_gateup(x, perm_token, offsets, sel, tile_start, max_tiles, bl
               _p(tile_start), int(max_tiles), int(block_m), _p(slots), H, I, _p(h_ws), _stream(dev))
 
 
+def swiglu_grouped_gateup_pair(x, perm_token, offsets, sel, tile_start_384, max_tiles_384, tile_start_256,
+                               max_tiles_256, slots, H, I, h_ws):
+    """The gate/up launch on 384-row or 256-row tiles, chosen on the device
+    from the two prefixes of one balanced order."""
+    dev = x.device
+    _need(x, "inputs", BF16, 2)
+    _need(h_ws, "h_ws", BF16, None, dev)
+    if h_ws.numel() < perm_token.numel() * I:
+        raise ValueError("h_ws is smaller than rows x I")
+    _lib.call("pdscope_swiglu_grouped_gateup_pair", _p(x), _p(perm_token), _p(offsets), _p(sel), sel.numel(),
+              _p(tile_start_384), int(max_tiles_384), _p(tile_start_256), int(max_tiles_256), _p(slots), H, I,
+              _p(h_ws), _stream(dev))
+
+
 def swiglu_grouped_down(h_ws, offsets, sel, tile_start, max_tiles, block_m, slots, H, I, y):
     """Only the down-projection launch of swiglu_grouped (K3, second half)."""
     dev = h_ws.device
