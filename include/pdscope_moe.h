@@ -208,16 +208,21 @@ int pdscope_swiglu_grouped_down(const void *h_ws, const int32_t *offsets, const 
                                 const void *const *slots, int H, int I, void *y, void *stream);
 
 /*
- * The gate/up half for 384-row or 256-row tiles, chosen on the device from
- * the two m-tile counts: tile_start_384 / tile_start_256 are the prefixes of
- * one balanced order (pdscope_schedule_balanced_pair and
- * pdscope_pack_schedule_balanced with block sizes 384 and 256), max_tiles_*
- * bound their last entries.  Limits: H % 256 == 0 and I % 128 == 0.
+ * Both halves with a row tile each (tile_start / max_tiles / block_m for
+ * gate/up, *_down for down, prefixes of one order `sel`), optionally with
+ * always-on shared experts as further tiles of the same two launches:
+ * h_shared [T, shared_I] and y_shared [T, H] bf16 receive the MLP
+ * shared_slot[0] (gate|up|down block of intermediate shared_I) over rows
+ * 0 .. T-1 of x (shared_slot NULL: none).  With block_m == 384 and
+ * block_m_down == 256 the gate/up launch takes whichever of the two row tiles
+ * suits the rows (chosen on the device; H % 256 == 0, I % 128 == 0).
  */
-int pdscope_swiglu_grouped_gateup_pair(const void *x, const int32_t *perm_token, const int32_t *offsets,
-                                       const int32_t *sel, int nsel, const int32_t *tile_start_384,
-                                       int max_tiles_384, const int32_t *tile_start_256, int max_tiles_256,
-                                       const void *const *slots, int H, int I, void *h_ws, void *stream);
+int pdscope_swiglu_grouped_layer(const void *x, const int32_t *perm_token, const int32_t *offsets,
+                                 const int32_t *sel, int nsel, const int32_t *tile_start, int max_tiles,
+                                 int block_m, const int32_t *tile_start_down, int max_tiles_down,
+                                 int block_m_down, const void *const *slots, int H, int I, void *h_ws, void *y,
+                                 int T, const void *const *shared_slot, int shared_I, void *h_shared,
+                                 void *y_shared, void *stream);
 
 /*
  * A8 fused weighted merge: replaces the index_add_ merge

@@ -39,8 +39,8 @@ SIGNATURES = {
     "pdscope_swiglu_grouped": ([_vp, _vp, _vp, _vp, _i32, _vp, _i32, _i32, _vp, _i32, _i32, _vp, _vp, _vp], _i32),
     "pdscope_swiglu_grouped_gateup": ([_vp, _vp, _vp, _vp, _i32, _vp, _i32, _i32, _vp, _i32, _i32, _vp, _vp], _i32),
     "pdscope_swiglu_grouped_down": ([_vp, _vp, _vp, _i32, _vp, _i32, _i32, _vp, _i32, _i32, _vp, _vp], _i32),
-    "pdscope_swiglu_grouped_gateup_pair": ([_vp, _vp, _vp, _vp, _i32, _vp, _i32, _vp, _i32, _vp, _i32, _i32, _vp,
-                                            _vp], _i32),
+    "pdscope_swiglu_grouped_layer": ([_vp, _vp, _vp, _vp, _i32, _vp, _i32, _i32, _vp, _i32, _i32, _vp, _i32, _i32,
+                                      _vp, _vp, _i32, _vp, _i32, _vp, _vp, _vp], _i32),
     "pdscope_merge": ([_vp, _vp, _vp, _i32, _i32, _i32, _vp, _vp, _vp], _i32),
     "pdscope_merge_ordered": ([_vp, _vp, _vp, _i32, _i32, _i32, _vp, _vp, _vp], _i32),
     "pdscope_swiglu_decode": ([_vp, _vp, _vp, _i32, _vp, _i32, _i32, _vp, _vp, _i32, _vp], _i32),

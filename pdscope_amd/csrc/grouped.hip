@@ -134,6 +134,21 @@ __device__ __forceinline__ void wait_stage(int younger) {
 // XCD b % 8): all n-tiles of an m-tile share the gathered activation rows
 // in one L2, and the m-tiles of one expert read the same weight tiles at
 // the same time from one L2.
+// Always-on shared experts as further tiles of a grouped launch (slot ==
+// nullptr: none): one MLP of intermediate I over rows 0 .. T-1 in order, on the
+// launch's own tile shape.  Its tiles take the first blocks of the grid: the
+// down half is the longest tile of the launch (K = shared I).  As launches of
+// their own on a second stream (48 blocks for the down half at T=1304) they
+// held CUs for long while the routed launches waited at the join, and their
+// time moved with how the two streams met (DeepSeek-V2-Lite layer, T=1304:
+// 320 to 360 us from run to run, 311 now; two layers of T=48 418 -> 398).
+struct SharedTiles {
+    const uint16_t *const *slot;  // [1] gate|up|down block
+    int I, T;
+    uint16_t *h;                  // [T, I]
+    uint16_t *y;                  // [T, H]
+};
+
 template <int BM, int BN, int BK, int SA, int SB>
 constexpr int kRingBytes = (SA * BM + SB * BN) * BK * 2;
 
@@ -141,8 +156,8 @@ template <int BM, int BN, int BK, int WM, int WN, int SA, int SB, bool ILV, bool
 __device__ __forceinline__ void grouped_tile(
     uint8_t *smem, const uint16_t *__restrict__ a_src, const int32_t *__restrict__ perm_token,
     const int32_t *__restrict__ offsets, const int32_t *__restrict__ sel, int nsel,
-    const int32_t *__restrict__ tile_start, const uint16_t *const *__restrict__ slots, int H, int I,
-    uint16_t *__restrict__ out) {
+    const int32_t *__restrict__ tile_start, const uint16_t *const *__restrict__ slots, int H, int I_routed,
+    uint16_t *__restrict__ out_routed, const SharedTiles &sh) {
     constexpr int NW = WM * WN;
     static_assert(NW == 4 || NW == 8, "4 or 8 waves");
     constexpr bool SPLIT = SA != SB;
@@ -162,34 +177,48 @@ __device__ __forceinline__ void grouped_tile(
     uint8_t *const ring_a = smem;
     uint8_t *const ring_b = smem + SA * ASTAGE;
 
-    // ---- tile -> (m-tile, n-tile)
+    // ---- tile -> (m-tile, n-tile): the shared tiles' blocks, then the routed ones'
+    const int nts = GATEUP ? sh.I / (BN / 2) : H / BN;
+    const int stotal = sh.slot ? (sh.T + BM - 1) / BM * nts : 0;
+    const int sblocks = (stotal + 7) & ~7;
+    const bool shared = (int)blockIdx.x < sblocks;
+    const int I = shared ? sh.I : I_routed;
     const int NT = GATEUP ? I / (BN / 2) : H / BN;
-    const int total = tile_start[nsel] * NT;
+    const int total = shared ? stotal : tile_start[nsel] * NT;
+    const int bid = shared ? blockIdx.x : blockIdx.x - sblocks;
     const int per_xcd = (total + 7) >> 3;
-    const int pos = blockIdx.x >> 3;
+    const int pos = bid >> 3;
     if (pos >= per_xcd) return;
-    const int t = (blockIdx.x & 7) * per_xcd + pos;
+    const int t = (bid & 7) * per_xcd + pos;
     if (t >= total) return;
     const int mt = t / NT, nt = t - mt * NT;
-    // the expert position of m-tile mt: the last lo with tile_start[lo] <= mt.
-    // tile_start is non-decreasing with tile_start[0] = 0, so lo is the count
-    // of j in [1, nsel) with tile_start[j] <= mt: independent loads and a
-    // ballot per 64 entries instead of a chain of dependent loads
-    int lo = 0;
+    int row0 = 0, row_end = sh.T, m0 = mt * BM;  // the expert's rows, the tile's first row
+    const uint16_t *base;
+    if (shared) {
+        base = sh.slot[0];
+    } else {
+        // the expert position of m-tile mt: the last lo with tile_start[lo] <= mt.
+        // tile_start is non-decreasing with tile_start[0] = 0, so lo is the count
+        // of j in [1, nsel) with tile_start[j] <= mt: independent loads and a
+        // ballot per 64 entries instead of a chain of dependent loads
+        int lo = 0;
 #pragma unroll 4
-    for (int base = 1; base < nsel; base += 64) {
-        const int j = base + (threadIdx.x & 63);
-        lo += __popcll(__ballot(j < nsel && tile_start[j] <= mt));
+        for (int b0 = 1; b0 < nsel; b0 += 64) {
+            const int j = b0 + (threadIdx.x & 63);
+            lo += __popcll(__ballot(j < nsel && tile_start[j] <= mt));
+        }
+        lo = __builtin_amdgcn_readfirstlane(lo);
+        const int e = sel[lo];
+        row0 = offsets[e];
+        row_end = offsets[e + 1];
+        m0 = row0 + (mt - tile_start[lo]) * BM;
+        base = slots[e];
     }
-    lo = __builtin_amdgcn_readfirstlane(lo);
-    const int e = sel[lo];
-    const int row_end = offsets[e + 1];
-    const int m0 = offsets[e] + (mt - tile_start[lo]) * BM;
     const int K = GATEUP ? H : I;
     const int n0 = nt * (GATEUP ? BN / 2 : BN);  // first intermediate (gate/up) or output column
-    const uint16_t *base = slots[e];
     if (base == nullptr) return;  // no ready copy of this expert: never dereference
     const size_t IH = (size_t)I * H;
+    uint16_t *const out = shared ? (GATEUP ? sh.h : sh.y) : out_routed;
 
     // ---- per-lane source rows: load q of A-wave wa covers A rows
     // RPI(wa + NWA q) .. +RPI-1 (B likewise with wb, NWB); lane l takes row
@@ -221,7 +250,7 @@ __device__ __forceinline__ void grouped_tile(
 #pragma unroll
         for (int q = 0; q < AL; ++q) {
             const int gr = min(m0 + (wa + NWA * q) * G::RPI + rl, row_end - 1);
-            lp[q] = (uint32_t)perm_token[gr] * (uint32_t)(H / 8) + a_cs;
+            lp[q] = (uint32_t)(shared ? gr : perm_token[gr]) * (uint32_t)(H / 8) + a_cs;
         }
     }
     // B: the lane's row and chunk in bytes from the first row of its load group
@@ -233,9 +262,9 @@ __device__ __forceinline__ void grouped_tile(
             return rb < BN / 2 ? (size_t)(n0 + rb) * H * 2 : (size_t)IH * 2 + (size_t)(n0 + rb - BN / 2) * H * 2;
         return (size_t)IH * 4 + (size_t)(n0 + rb) * I * 2;
     };
-    const uint8_t *const a_base = reinterpret_cast<const uint8_t *>(a_src);
+    const uint8_t *const a_base = reinterpret_cast<const uint8_t *>(shared && !GATEUP ? sh.h : a_src);
     const uint8_t *const b_base = reinterpret_cast<const uint8_t *>(base);
-    const bool one_tile = row_end - offsets[e] <= BM;  // no other m-tile reads these weights
+    const bool one_tile = row_end - row0 <= BM;  // no other m-tile reads these weights
     const int KT = K / BK;
     auto issue_a = [&](int kt) __attribute__((always_inline)) {
         uint8_t *st = ring_a + (kt % SA) * ASTAGE;
@@ -509,10 +538,10 @@ __global__ __launch_bounds__(64 * WM * WN, OCC == 1 ? 1 : OCC * WM * WN / 4) voi
     const uint16_t *__restrict__ a_src, const int32_t *__restrict__ perm_token,
     const int32_t *__restrict__ offsets, const int32_t *__restrict__ sel, int nsel,
     const int32_t *__restrict__ tile_start, const uint16_t *const *__restrict__ slots, int H, int I,
-    uint16_t *__restrict__ out) {
+    uint16_t *__restrict__ out, SharedTiles sh) {
     __shared__ __attribute__((aligned(1024))) uint8_t smem[kRingBytes<BM, BN, BK, SA, SB>];
     grouped_tile<BM, BN, BK, WM, WN, SA, SB, ILV, GATEUP, OCC, FK>(smem, a_src, perm_token, offsets, sel, nsel,
-                                                                   tile_start, slots, H, I, out);
+                                                                   tile_start, slots, H, I, out, sh);
 }
 
 // Gate/up for a mean of about 200..320 rows per expert, where the better tile
@@ -529,95 +558,100 @@ __global__ __launch_bounds__(512, 1) void grouped_gateup_pair_kernel(
     const uint16_t *__restrict__ x, const int32_t *__restrict__ perm_token, const int32_t *__restrict__ offsets,
     const int32_t *__restrict__ sel, int nsel, const int32_t *__restrict__ tile_start_384,
     const int32_t *__restrict__ tile_start_256, const uint16_t *const *__restrict__ slots, int H, int I,
-    uint16_t *__restrict__ h_ws) {
+    uint16_t *__restrict__ h_ws, SharedTiles sh) {
     constexpr int B384 = kRingBytes<384, 128, 64, 2, 4>, B256 = kRingBytes<256, 256, 64, 2, 3>;
     __shared__ __attribute__((aligned(1024))) uint8_t smem[B384 > B256 ? B384 : B256];
     const int m384 = tile_start_384[nsel], m256 = tile_start_256[nsel];
     if (4 * m384 <= 3 * m256)
         grouped_tile<384, 128, 64, 4, 2, 2, 4, true, true, 1, 32>(smem, x, perm_token, offsets, sel, nsel,
-                                                                  tile_start_384, slots, H, I, h_ws);
+                                                                  tile_start_384, slots, H, I, h_ws, sh);
     else
         grouped_tile<256, 256, 64, 2, 4, 2, 3, true, true, 1, 16>(smem, x, perm_token, offsets, sel, nsel,
-                                                                  tile_start_256, slots, H, I, h_ws);
+                                                                  tile_start_256, slots, H, I, h_ws, sh);
+}
+
+// Everything a grouped launch takes beside its tile configuration.
+struct GroupedArgs {
+    const uint16_t *x;
+    const int32_t *perm_token, *offsets, *sel;
+    int nsel;
+    const int32_t *tile_start;
+    int max_tiles;
+    const uint16_t *const *slots;
+    int H, I;
+    uint16_t *h_ws, *y;
+    SharedTiles sh;
+    hipStream_t s;
+};
+
+// Blocks of a launch: the shared tiles', then every (m-tile, n-tile) the bound
+// allows, each a multiple of 8 so each XCD's contiguous piece of a tile range
+// has blocks.
+static unsigned grouped_grid(const GroupedArgs &a, int max_tiles, int BM, int nt, int nt_shared) {
+    const size_t shared = a.sh.slot ? (size_t)((a.sh.T + BM - 1) / BM) * (size_t)nt_shared : 0;
+    return (unsigned)((shared + 7) / 8 * 8 + ((size_t)max_tiles * (size_t)nt + 7) / 8 * 8);
 }
 
 // phase: 1 = gate/up only, 2 = down only, 3 = both
 // PH: the phases (1 gate/up, 2 down) this tile configuration serves
 template <int BM, int BN, int BK, int WM, int WN, int SA, int SB, bool ILV = false, int PH = 3, int OCC = 1,
           int FK = 32>
-int launch_grouped(int phase, const uint16_t *x, const int32_t *perm_token, const int32_t *offsets,
-                   const int32_t *sel, int nsel, const int32_t *tile_start, int max_tiles,
-                   const uint16_t *const *slots, int H, int I, uint16_t *h_ws, uint16_t *y, hipStream_t s) {
-    if (I % (BN / 2) || H % BN || H % BK || I % BK)
+int launch_grouped(int phase, const GroupedArgs &a) {
+    if (a.I % (BN / 2) || a.H % BN || a.H % BK || a.I % BK)
         return fail(kEInval, "grouped: I must divide by BN/2, H by BN, and both by the K step");
-    // grid: every (m-tile, n-tile) the bound allows, a multiple of 8 so each
-    // XCD's contiguous piece of the tile range has blocks
+    if (a.sh.slot && (a.sh.I % (BN / 2) || a.sh.I % BK))
+        return fail(kEInval, "grouped: the shared I must divide by BN/2 and the K step");
     if constexpr ((PH & 1) != 0) if (phase & 1) {
-        const size_t n1 = (size_t)max_tiles * (size_t)(I / (BN / 2));
-        const unsigned g1 = (unsigned)((n1 + 7) / 8 * 8);
-        grouped_kernel<BM, BN, BK, WM, WN, SA, SB, ILV, true, OCC, FK><<<g1, 64 * WM * WN, 0, s>>>(x, perm_token, offsets, sel, nsel, tile_start,
-                                                                    slots, H, I, h_ws);
+        grouped_kernel<BM, BN, BK, WM, WN, SA, SB, ILV, true, OCC, FK>
+            <<<grouped_grid(a, a.max_tiles, BM, a.I / (BN / 2), a.sh.I / (BN / 2)), 64 * WM * WN, 0, a.s>>>(
+                a.x, a.perm_token, a.offsets, a.sel, a.nsel, a.tile_start, a.slots, a.H, a.I, a.h_ws, a.sh);
         int rc = check_launch("grouped_kernel<gateup>");
         if (rc) return rc;
     }
     if constexpr ((PH & 2) != 0) if (phase & 2) {
-        const size_t n2 = (size_t)max_tiles * (size_t)(H / BN);
-        const unsigned g2 = (unsigned)((n2 + 7) / 8 * 8);
-        grouped_kernel<BM, BN, BK, WM, WN, SA, SB, ILV, false, OCC, FK><<<g2, 64 * WM * WN, 0, s>>>(h_ws, nullptr, offsets, sel, nsel, tile_start,
-                                                                     slots, H, I, y);
+        grouped_kernel<BM, BN, BK, WM, WN, SA, SB, ILV, false, OCC, FK>
+            <<<grouped_grid(a, a.max_tiles, BM, a.H / BN, a.H / BN), 64 * WM * WN, 0, a.s>>>(
+                a.h_ws, nullptr, a.offsets, a.sel, a.nsel, a.tile_start, a.slots, a.H, a.I, a.y, a.sh);
         return check_launch("grouped_kernel<down>");
     }
     return kOk;
 }
 
-int grouped_entry(int phase, const void *x, const int32_t *perm_token, const int32_t *offsets, const int32_t *sel,
-                  int nsel, const int32_t *tile_start, int max_tiles, int block_m, const void *const *slots, int H,
-                  int I, void *h_ws, void *y, void *stream) {
-    if (((phase & 1) && (!x || !perm_token)) || !offsets || !sel || !tile_start || !slots || !h_ws ||
-        ((phase & 2) && !y))
+static int grouped_check(int phase, int block_m, const GroupedArgs &a) {
+    if (((phase & 1) && (!a.x || !a.perm_token)) || !a.offsets || !a.sel || !a.tile_start || !a.slots || !a.h_ws ||
+        ((phase & 2) && !a.y))
         return fail(kEInval, "grouped: null pointer");
-    if (nsel < 1 || max_tiles < 1) return fail(kEInval, "grouped: need nsel >= 1 and max_tiles >= 1");
-    if (H % 64 || I % 64 || H < 64 || I < 64) return fail(kEInval, "grouped: need H % 64 == 0 and I % 64 == 0");
-    if (max_tiles > (1 << 22)) return fail(kEInval, "grouped: max_tiles too large");
-    hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-    const uint16_t *xp = (const uint16_t *)x;
-    const uint16_t *const *sp = (const uint16_t *const *)slots;
+    if (a.nsel < 1 || a.max_tiles < 1) return fail(kEInval, "grouped: need nsel >= 1 and max_tiles >= 1");
+    if (a.H % 64 || a.I % 64 || a.H < 64 || a.I < 64)
+        return fail(kEInval, "grouped: need H % 64 == 0 and I % 64 == 0");
+    if (a.max_tiles > (1 << 22)) return fail(kEInval, "grouped: max_tiles too large");
+    if (a.sh.slot && (a.sh.I < 64 || a.sh.T < 1 || !a.sh.h || !a.sh.y))
+        return fail(kEInval, "grouped: bad shared arguments");
+    if (block_m == 32 && a.H % 256) return fail(kEInval, "grouped: H must divide by 256");
+    return kOk;
+}
+
+static int grouped_phase(int phase, int block_m, const GroupedArgs &a) {
+    int rc = grouped_check(phase, block_m, a);
+    if (rc != kOk) return rc;
     switch (block_m) {
-    case 32: {
+    case 32:
         // down (K = I, a short K loop): two workgroups of 128 columns per CU, so
         // that one's ring fill and epilogue overlap the other's loads (T=201:
         // 71 -> 67 us, T=17: 46.8 -> 44.5); gate/up is faster on 256 columns
         // and a CU of its own (T=201: 128 us against 136 at two per CU)
-        if (H % 256) return fail(kEInval, "grouped: H must divide by 256");
-        int rc = kOk;
-        if (phase & 1)
-            rc = launch_grouped<32, 256, 64, 1, 4, 4, 4, false, 1>(1, xp, perm_token, offsets, sel, nsel, tile_start,
-                                                                   max_tiles, sp, H, I, (uint16_t *)h_ws,
-                                                                   (uint16_t *)y, s);
-        if (rc == kOk && (phase & 2))
-            rc = launch_grouped<32, 128, 64, 1, 4, 4, 4, false, 2, 2>(2, xp, perm_token, offsets, sel, nsel, tile_start,
-                                                                      max_tiles, sp, H, I, (uint16_t *)h_ws,
-                                                                      (uint16_t *)y, s);
+        if (phase & 1) rc = launch_grouped<32, 256, 64, 1, 4, 4, 4, false, 1>(1, a);
+        if (rc == kOk && (phase & 2)) rc = launch_grouped<32, 128, 64, 1, 4, 4, 4, false, 2, 2>(2, a);
         return rc;
-    }
-    case 64: {
+    case 64:
         // gate/up: split load roles, 3 + 4 stages, one workgroup per CU; down
         // (K = I, a short K loop): every wave loads both operands, 2 + 2
         // stages, two workgroups per CU (T=512: 79.6 against 85.3 us)
-        int rc = kOk;
-        if (phase & 1)
-            rc = launch_grouped<64, 256, 64, 2, 4, 3, 4, false, 1>(1, xp, perm_token, offsets, sel, nsel, tile_start,
-                                                                   max_tiles, sp, H, I, (uint16_t *)h_ws,
-                                                                   (uint16_t *)y, s);
-        if (rc == kOk && (phase & 2))
-            rc = launch_grouped<64, 256, 64, 2, 4, 2, 2, false, 2, 2>(2, xp, perm_token, offsets, sel, nsel, tile_start,
-                                                                      max_tiles, sp, H, I, (uint16_t *)h_ws,
-                                                                      (uint16_t *)y, s);
+        if (phase & 1) rc = launch_grouped<64, 256, 64, 2, 4, 3, 4, false, 1>(1, a);
+        if (rc == kOk && (phase & 2)) rc = launch_grouped<64, 256, 64, 2, 4, 2, 2, false, 2, 2>(2, a);
         return rc;
-    }
     case 128:
-        return launch_grouped<128, 256, 64, 2, 4, 3, 3>(phase, xp, perm_token, offsets, sel, nsel, tile_start, max_tiles,
-                                                 sp, H, I, (uint16_t *)h_ws, (uint16_t *)y, s);
+        return launch_grouped<128, 256, 64, 2, 4, 3, 3>(phase, a);
     case 256:
         // 128-byte row pieces (BK 64) halve the L2 requests of the 64-byte
         // ones; each CU keeps about 64 requests in flight, so the bytes per
@@ -629,15 +663,22 @@ int grouped_entry(int phase, const void *x, const int32_t *perm_token, const int
         // 32-row blocks dealt to the two wave rows in turn: an expert of fewer
         // rows than the tile keeps both busy (T=2048, 128 rows each: gate/up
         // 163 -> 153 us, down 96 -> 90; T=4096 Zipf down 173 -> 162)
-        return launch_grouped<256, 256, 64, 2, 4, 2, 3, true, 3, 1, 16>(phase, xp, perm_token, offsets, sel, nsel,
-                                                                         tile_start, max_tiles, sp, H, I,
-                                                                         (uint16_t *)h_ws, (uint16_t *)y, s);
+        return launch_grouped<256, 256, 64, 2, 4, 2, 3, true, 3, 1, 16>(phase, a);
     case 384:
-        return launch_grouped<384, 128, 64, 4, 2, 2, 4, true>(phase, xp, perm_token, offsets, sel, nsel, tile_start,
-                                                       max_tiles, sp, H, I, (uint16_t *)h_ws, (uint16_t *)y, s);
+        return launch_grouped<384, 128, 64, 4, 2, 2, 4, true>(phase, a);
     default:
         return fail(kEInval, "grouped: block_m must be 32, 64, 128, 256 or 384");
     }
+}
+
+static int grouped_entry(int phase, const void *x, const int32_t *perm_token, const int32_t *offsets,
+                         const int32_t *sel, int nsel, const int32_t *tile_start, int max_tiles, int block_m,
+                         const void *const *slots, int H, int I, void *h_ws, void *y, void *stream) {
+    return grouped_phase(phase, block_m,
+                         GroupedArgs{(const uint16_t *)x, perm_token, offsets, sel, nsel, tile_start, max_tiles,
+                                     (const uint16_t *const *)slots, H, I, (uint16_t *)h_ws, (uint16_t *)y,
+                                     SharedTiles{nullptr, 0, 0, nullptr, nullptr},
+                                     reinterpret_cast<hipStream_t>(stream)});
 }
 
 }  // namespace pd
@@ -684,22 +725,35 @@ PD_API int pdscope_swiglu_grouped_gateup(const void *x, const int32_t *perm_toke
                          nullptr, stream);
 }
 
-PD_API int pdscope_swiglu_grouped_gateup_pair(const void *x, const int32_t *perm_token, const int32_t *offsets,
-                                              const int32_t *sel, int nsel, const int32_t *tile_start_384,
-                                              int max_tiles_384, const int32_t *tile_start_256, int max_tiles_256,
-                                              const void *const *slots, int H, int I, void *h_ws, void *stream) {
-    if (!x || !perm_token || !offsets || !sel || !tile_start_384 || !tile_start_256 || !slots || !h_ws)
-        return fail(kEInval, "grouped: null pointer");
-    if (nsel < 1 || max_tiles_384 < 1 || max_tiles_256 < 1)
-        return fail(kEInval, "grouped: need nsel >= 1 and max_tiles >= 1");
-    if (H % 256 || I % 128 || H < 256 || I < 128)
+PD_API int pdscope_swiglu_grouped_layer(const void *x, const int32_t *perm_token, const int32_t *offsets,
+                                        const int32_t *sel, int nsel, const int32_t *tile_start, int max_tiles,
+                                        int block_m, const int32_t *tile_start_down, int max_tiles_down,
+                                        int block_m_down, const void *const *slots, int H, int I, void *h_ws, void *y,
+                                        int T, const void *const *shared_slot, int shared_I, void *h_shared,
+                                        void *y_shared, void *stream) {
+    const SharedTiles sh = {(const uint16_t *const *)shared_slot, shared_slot ? shared_I : 0, T, (uint16_t *)h_shared,
+                            (uint16_t *)y_shared};
+    GroupedArgs a{(const uint16_t *)x, perm_token, offsets, sel, nsel, tile_start, max_tiles,
+                  (const uint16_t *const *)slots, H, I, (uint16_t *)h_ws, (uint16_t *)y, sh,
+                  reinterpret_cast<hipStream_t>(stream)};
+    GroupedArgs d = a;
+    d.tile_start = tile_start_down;
+    d.max_tiles = max_tiles_down;
+    if (block_m != 384 || block_m_down != 256) {
+        const int rc = grouped_phase(1, block_m, a);
+        return rc != kOk ? rc : grouped_phase(2, block_m_down, d);
+    }
+    int rc = grouped_check(3, 384, a);
+    if (rc == kOk) rc = grouped_check(3, 256, d);
+    if (rc != kOk) return rc;
+    if (H % 256 || I % 128 || sh.I % 128)
         return fail(kEInval, "grouped: the tile pair needs H % 256 == 0 and I % 128 == 0");
-    if (max_tiles_384 > (1 << 22) || max_tiles_256 > (1 << 22)) return fail(kEInval, "grouped: max_tiles too large");
-    const size_t n = std::max((size_t)max_tiles_384 * (size_t)(I / 64), (size_t)max_tiles_256 * (size_t)(I / 128));
-    grouped_gateup_pair_kernel<<<(unsigned)((n + 7) / 8 * 8), 512, 0, reinterpret_cast<hipStream_t>(stream)>>>(
-        (const uint16_t *)x, perm_token, offsets, sel, nsel, tile_start_384, tile_start_256,
-        (const uint16_t *const *)slots, H, I, (uint16_t *)h_ws);
-    return check_launch("grouped_gateup_pair_kernel");
+    const unsigned grid = std::max(grouped_grid(a, max_tiles, 384, I / 64, sh.I / 64),
+                                   grouped_grid(d, max_tiles_down, 256, I / 128, sh.I / 128));
+    grouped_gateup_pair_kernel<<<grid, 512, 0, a.s>>>(a.x, perm_token, offsets, sel, nsel, tile_start, tile_start_down,
+                                                      a.slots, H, I, a.h_ws, sh);
+    rc = check_launch("grouped_gateup_pair_kernel");
+    return rc != kOk ? rc : grouped_phase(2, 256, d);
 }
 
 PD_API int pdscope_swiglu_grouped_down(const void *h_ws, const int32_t *offsets, const int32_t *sel, int nsel,

@@ -108,13 +108,19 @@ def decode_shared_fits(ws: MoEWorkspace) -> bool:
             and ops.decode_shared_supported(ws.H, ws.I, ws.E, ws.k, ws.shared_I))
 
 
+def shared_in_grouped(ws: MoEWorkspace) -> bool:
+    """Whether shared experts run as tiles of the routed experts' own grouped
+    launches (any of their row tiles); other shapes take launches of their
+    own on the side stream."""
+    return ws.shared_I % 128 == 0 and ws.I % 128 == 0 and ws.H % 256 == 0
+
+
 def shared_block_m(T: int, I: int) -> int:
-    """Row-tile height of the shared experts' launch.  It runs on a side
-    stream beside the routing and the routed experts, so it should read its
-    weights as few times as possible and hold few CUs while the small routing
-    and pack launches run: the tallest tile the shape allows (DeepSeek-V2-Lite
-    mixed batch of 1304 tokens: 353 us per layer on 256-row tiles against
-    376 us on 64-row tiles sized to fill the device alone, bit-identical)."""
+    """Row-tile height of the shared experts' own launch, for shapes whose
+    shared tiles cannot join the grouped launches.  It runs on a side stream
+    beside the routing and the routed experts, so it should read its weights as
+    few times as possible and hold few CUs while the small routing and pack
+    launches run: the tallest tile the shape allows."""
     if I % _GATEUP_COLS[256] != 0:
         return 384
     return 32 if T <= 16 else 256
@@ -139,16 +145,18 @@ def shared_forward(x, shared_slot, ws: MoEWorkspace):
 
 
 def experts_resident(x, ids, weights, slots, ws: MoEWorkspace, out=None, *, block_m=None, add_in=None,
-                     merge="fused", before_merge=None):
+                     merge="fused", before_merge=None, shared_slot=None):
     """K4 (T == 1) or K2+K3+K5 (T > 1) over experts that are all addressable in `slots`.
     add_in [T, H] bf16 (shared-expert output) is added unweighted in the merge;
     before_merge() runs right before the merge is enqueued (to order add_in's producer).
+    shared_slot (int64 [1], T > 1, shared_in_grouped(ws)): shared experts run as
+    further tiles of the grouped launches, into ws.y_shared, and are added in the merge.
     merge: 'fused' (fp32 sum, one rounding) or 'reference' (bf16 adds in
     ascending expert id, the reference runtime's default merge)."""
     T = x.shape[0]
     H, I, E, k = ws.H, ws.I, ws.E, ws.k
     out = ws.out[:T] if out is None else out
-    if T == 1 and add_in is None:
+    if T == 1 and add_in is None and shared_slot is None:
         ops.swiglu_decode(x, ids, weights, slots, H, I, ws.h_ws, out, merge=merge)
         return out
     _, _, _, packed = ws.views(T)
@@ -158,7 +166,9 @@ def experts_resident(x, ids, weights, slots, ws: MoEWorkspace, out=None, *, bloc
     sched = (ws.sel_all, bm, ws.sel_order, ws.tile_start) + ((bmd, ws.tile_start_down) if bmd != bm else ())
     ops.pack(ids, E, out=packed, workspace=ws.pack_ws, schedule=sched)
     grouped_ffn(x, packed, ws.sel_all, bm, (T * k + bm - 1) // bm + E, slots, ws,
-                max_tiles_down=(T * k + bmd - 1) // bmd + E, scheduled=True)
+                max_tiles_down=(T * k + bmd - 1) // bmd + E, scheduled=True, shared_slot=shared_slot)
+    if shared_slot is not None:
+        add_in = ws.y_shared[:T]
     if before_merge is not None:
         before_merge()
     ops.merge(ws.y, packed.row_of, weights, out, add_in=add_in, mode=merge)
@@ -176,30 +186,31 @@ def down_block_m(bm: int, H: int, I: int) -> int:
 
 
 def grouped_ffn(x, packed, sel, bm, max_tiles, slots, ws: MoEWorkspace, *, max_tiles_down, perm=None,
-                scheduled=False):
+                scheduled=False, shared_slot=None):
     """Grouped SwiGLU over the experts in `sel` (int32 device): gate/up on
     bm-row tiles into ws.h_ws, down on down_block_m(bm, H, I)-row tiles into ws.y.
     max_tiles / max_tiles_down bound the two launches' tile counts.  perm
     (default packed.perm_token) maps grouped rows to rows of x.  scheduled:
     ws.sel_order / ws.tile_start (/ ws.tile_start_down) already hold the
-    balanced schedule of `sel` (written by the pack launch)."""
+    balanced schedule of `sel` (written by the pack launch).  shared_slot:
+    shared experts over every row of x as further tiles of both launches."""
     H, I = ws.H, ws.I
     perm = packed.perm_token if perm is None else perm
     nsel = sel.numel()
     tile_start, order = ws.tile_start[:nsel + 1], ws.sel_order[:nsel]
     bmd = down_block_m(bm, H, I)
     if bmd == bm:
+        tile_down, max_tiles_down = tile_start, max_tiles
         if not scheduled:
             ops.schedule(packed.counts, sel, bm, out=tile_start, order=order)
-        ops.swiglu_grouped(x, perm, packed.offsets, order, tile_start, max_tiles, bm, slots, H, I, ws.h_ws, ws.y)
-        return
-    # one launch schedules both: the balanced order depends on the rows only
-    tile_down = ws.tile_start_down[:nsel + 1]
-    if not scheduled:
-        ops.schedule(packed.counts, sel, bm, out=tile_start, order=order, block_m2=bmd, out2=tile_down)
-    ops.swiglu_grouped_gateup_pair(x, perm, packed.offsets, order, tile_start, max_tiles, tile_down, max_tiles_down,
-                                   slots, H, I, ws.h_ws)
-    ops.swiglu_grouped_down(ws.h_ws, packed.offsets, order, tile_down, max_tiles_down, bmd, slots, H, I, ws.y)
+    else:
+        # one launch schedules both: the balanced order depends on the rows only
+        tile_down = ws.tile_start_down[:nsel + 1]
+        if not scheduled:
+            ops.schedule(packed.counts, sel, bm, out=tile_start, order=order, block_m2=bmd, out2=tile_down)
+    shared = None if shared_slot is None else (shared_slot, ws.shared_I, ws.h_shared, ws.y_shared)
+    ops.swiglu_grouped_layer(x, perm, packed.offsets, order, tile_start, max_tiles, bm, tile_down, max_tiles_down, bmd,
+                             slots, H, I, ws.h_ws, ws.y, shared=shared)
 
 
 def moe_forward(x, gate, slots, ws: MoEWorkspace, *, normalize=True, bias=None, block_m=None, fused_decode=True,
@@ -230,6 +241,10 @@ def moe_forward(x, gate, slots, ws: MoEWorkspace, *, normalize=True, bias=None, 
                                     out=out, logits=logits, ids=ids, weights=weights, h_ws=ws.h_ws,
                                     h_shared=ws.h_shared, y_shared=ws.y_shared[:1], workspace=ws.route_ws,
                                     merge=merge)
+            return out, logits, ids, weights
+        if shared_in_grouped(ws):
+            logits, ids, weights = route(x, gate, ws, normalize=normalize, bias=bias)
+            out = experts_resident(x, ids, weights, slots, ws, block_m=block_m, merge=merge, shared_slot=shared_slot)
             return out, logits, ids, weights
         # the shared experts need only x: they run on a side stream beside the
         # routing and the routed experts (a one-expert launch alone does not

@@ -267,18 +267,34 @@ def swiglu_grouped_gateup(x, perm_token, offsets, sel, tile_start, max_tiles, bl
               _p(tile_start), int(max_tiles), int(block_m), _p(slots), H, I, _p(h_ws), _stream(dev))
 
 
-def swiglu_grouped_gateup_pair(x, perm_token, offsets, sel, tile_start_384, max_tiles_384, tile_start_256,
-                               max_tiles_256, slots, H, I, h_ws):
-    """The gate/up launch on 384-row or 256-row tiles, chosen on the device
-    from the two prefixes of one balanced order."""
-    dev = x.device
+def swiglu_grouped_layer(x, perm_token, offsets, sel, tile_start, max_tiles, block_m, tile_start_down, max_tiles_down,
+                         block_m_down, slots, H, I, h_ws, y, *, shared=None):
+    """Gate/up and down launches with a row tile each; shared=(slot, shared_I,
+    h_shared, y_shared) adds always-on shared experts over all rows of x to
+    the same two launches (see pdscope_swiglu_grouped_layer)."""
     _need(x, "inputs", BF16, 2)
+    dev = x.device
+    for t, n in ((perm_token, "perm_token"), (offsets, "offsets"), (sel, "sel"), (tile_start, "tile_start"),
+                 (tile_start_down, "tile_start_down")):
+        _need(t, n, torch.int32, 1, dev)
+    _need(slots, "slots", torch.int64, 1, dev)
     _need(h_ws, "h_ws", BF16, None, dev)
-    if h_ws.numel() < perm_token.numel() * I:
-        raise ValueError("h_ws is smaller than rows x I")
-    _lib.call("pdscope_swiglu_grouped_gateup_pair", _p(x), _p(perm_token), _p(offsets), _p(sel), sel.numel(),
-              _p(tile_start_384), int(max_tiles_384), _p(tile_start_256), int(max_tiles_256), _p(slots), H, I,
-              _p(h_ws), _stream(dev))
+    _need(y, "y", BF16, None, dev)
+    if h_ws.numel() < perm_token.numel() * I or y.numel() < perm_token.numel() * H:
+        raise ValueError("h_ws / y workspaces are smaller than rows x I / rows x H")
+    slot, shared_I, h_shared, y_shared = shared if shared is not None else (None, 0, None, None)
+    T = x.shape[0]
+    if slot is not None:
+        _need(slot, "shared_slot", torch.int64, 1, dev)
+        _need(h_shared, "h_shared", BF16, None, dev)
+        _need(y_shared, "y_shared", BF16, None, dev)
+        if x.shape[1] != H or h_shared.numel() < T * shared_I or y_shared.numel() < T * H:
+            raise ValueError("h_shared / y_shared must hold T rows of shared_I / H values")
+    _lib.call("pdscope_swiglu_grouped_layer", _p(x), _p(perm_token), _p(offsets), _p(sel), sel.numel(),
+              _p(tile_start), int(max_tiles), int(block_m), _p(tile_start_down), int(max_tiles_down),
+              int(block_m_down), _p(slots), H, I, _p(h_ws), _p(y), T, _p(slot), shared_I, _p(h_shared), _p(y_shared),
+              _stream(dev))
+    return y
 
 
 def swiglu_grouped_down(h_ws, offsets, sel, tile_start, max_tiles, block_m, slots, H, I, y):

@@ -621,3 +621,51 @@ def test_deepseek_v2_lite_layer_with_shared_experts(orc, pd):
     ref = orc.merge(y_ref, p["row_of"], wk, add_in=shared_ref)
     m = err_metrics(orc.bf16_to_f32(u16(out)), orc.bf16_to_f32(ref))
     assert m["max_rel"] <= MAX_REL and m["mean_abs"] <= MEAN_ABS, m
+
+
+@pytest.mark.parametrize("T,bm,bmd,skew", [(1, 32, 32, False), (33, 32, 32, True), (65, 64, 64, False),
+                                           (129, 128, 128, True), (255, 256, 256, False), (257, 384, 256, False),
+                                           (700, 384, 256, True), (385, 384, 384, False)])
+def test_grouped_layer_tiles_equal_the_plain_launches(pd, T, bm, bmd, skew):
+    """swiglu_grouped_layer (a row tile per half, the 384/256 choice on the
+    device on both sides of its rule, shared experts as further tiles) gives
+    the bits of the plain launches: every row is the same arithmetic in every
+    tile.  T around the tile heights, so the shared rows end inside a tile."""
+    ops, layer, synthetic = pd
+    H, I, E, k, Is = 256, 128, 32, 4, 384
+    lay = synthetic.make_layer(H, I, E, k, True, seed=T, device=DEV, shared_I=Is)
+    x = synthetic.make_tokens(T, H, seed=T + 1, device=DEV)
+    bias = synthetic.zipf_bias(E, 1.5, seed=2, device=DEV)[0] if skew else None
+    slots = ops.slot_table([lay.experts[e] for e in range(E)], DEV)
+    shared = ops.slot_table([lay.shared], DEV)
+    ws = layer.MoEWorkspace(T, H, I, E, k, DEV, shared_I=Is)
+    _, ids, _ = layer.route(x, lay.gate, ws, bias=bias)
+    n = T * k
+    packed = ops.pack(ids, E)
+    sel = torch.arange(E, dtype=torch.int32, device=DEV)
+
+    def tiles(b):
+        order = torch.empty_like(sel)
+        return order, ops.schedule(packed.counts, sel, b, order=order), (n + b - 1) // b + E
+
+    def bufs(rows, inner):
+        return (torch.full((rows * inner,), 7.0, dtype=torch.bfloat16, device=DEV),
+                torch.full((rows * H,), 7.0, dtype=torch.bfloat16, device=DEV))
+
+    order, ts, mt = tiles(64)
+    ref_h, ref_y = bufs(n, I)
+    ops.swiglu_grouped(x, packed.perm_token, packed.offsets, order, ts, mt, 64, slots, H, I, ref_h, ref_y)
+    one = dict(dtype=torch.int32, device=DEV)
+    ref_hs, ref_ys = bufs(T, Is)
+    ops.swiglu_grouped(x, torch.arange(T, **one), torch.tensor([0, T], **one), torch.zeros(1, **one),
+                       torch.tensor([0, (T + 63) // 64], **one), (T + 63) // 64, 64, shared, H, Is, ref_hs, ref_ys)
+    (order, ts, mt), (_, tsd, mtd) = tiles(bm), tiles(bmd)
+    for with_shared in (False, True):
+        h, y = bufs(n, I)
+        hs, ys = bufs(T, Is)
+        ops.swiglu_grouped_layer(x, packed.perm_token, packed.offsets, order, ts, mt, bm, tsd, mtd, bmd, slots, H, I,
+                                 h, y, shared=(shared, Is, hs, ys) if with_shared else None)
+        torch.cuda.synchronize()
+        assert torch.equal(h, ref_h) and torch.equal(y, ref_y)
+        if with_shared:
+            assert torch.equal(hs, ref_hs) and torch.equal(ys, ref_ys)
