@@ -37,6 +37,7 @@ from __future__ import annotations
 
 import bisect
 import itertools
+import operator
 from collections import Counter
 from collections.abc import Mapping
 from dataclasses import dataclass, field
@@ -234,14 +235,9 @@ class _Reveal:
     open_keys: set
 
 
-def _order(key):
-    """ExpertKey order as a plain tuple (the dataclass orders by these fields
-    in this order): sorting and bisecting on it compares in C."""
-    return key._t
-
-
-def _order_item(item):
-    return _order(item[0])
+# ExpertKey order as a plain tuple (the dataclass orders by these fields in
+# this order): sorting and bisecting on it compares in C
+_fields = operator.attrgetter("_t")
 
 
 class _Ranking:
@@ -272,7 +268,7 @@ class _Ranking:
         if bucket is None:
             bucket = self._buckets[rank] = []
             bisect.insort(self._ranks, rank)
-        t = key._t   # _order(key), inline on this path
+        t = key._t   # _fields(key), inline on this path
         bisect.insort(bucket, t)
         self._key_of[t] = key
         rank_of[key] = rank
@@ -303,6 +299,32 @@ class _Ranking:
         if not bucket:
             del self._buckets[rank]
             del self._ranks[bisect.bisect_left(self._ranks, rank)]
+
+    def discard_many(self, keys):
+        """discard(key) of each key; a rank's bucket that loses several keys is
+        emptied or filtered in one pass."""
+        rank_of, key_of, gone = self._rank_of, self._key_of, {}
+        for key in keys:
+            rank = rank_of.pop(key, None)
+            if rank is not None:
+                t = key._t
+                del key_of[t]
+                ts = gone.get(rank)
+                if ts is None:
+                    gone[rank] = [t]
+                else:
+                    ts.append(t)
+        for rank, ts in gone.items():
+            bucket = self._buckets[rank]
+            if len(ts) == len(bucket):
+                del self._buckets[rank]
+                del self._ranks[bisect.bisect_left(self._ranks, rank)]
+            elif len(ts) < 4:
+                for t in ts:
+                    del bucket[bisect.bisect_left(bucket, t)]
+            else:
+                drop = set(ts)
+                bucket[:] = [t for t in bucket if t not in drop]
 
     def ascending(self):
         for rank in list(self._ranks):
@@ -423,7 +445,7 @@ class ExpertCache:
 
     @property
     def unfinished_demand_keys(self):
-        return () if self._reveal is None else tuple(sorted(self._reveal.open_keys, key=_order))
+        return () if self._reveal is None else tuple(sorted(self._reveal.open_keys, key=_fields))
 
     @property
     def retention_hint(self):
@@ -509,23 +531,29 @@ class ExpertCache:
         bucket in one pass instead of one insertion each."""
         ranked, copies, r, hint = self._ranked, self._copies, self._reveal, self._hint
         replacing, lfu = self.policy != "static", self.policy == "LFU"
+        protected, hinted, last_get = self._protected, hint.keys if hint is not None else (), self._last_tick.get
+        open_keys = r.open_keys if r is not None else ()
+        unprotected, kept = self._unprotected, self._protected_rank
         groups = {}
+        at = members = None   # the group of the key before: neighbours mostly share it
         for key in keys:
             if key in ranked:
                 self._reindex(key)
                 continue
             c = copies.get(key)
             if (c is None or not replacing or c.ticket.pool != "cache" or c.phase != READY or c.holders
-                    or (r is not None and key in r.open_keys)):
+                    or key in open_keys):
                 continue
-            target = (self._protected_rank if key in self._protected or (hint is not None and key in hint.keys)
-                      else self._unprotected)
-            tick = self._last_tick.get(key, 0)
-            rank = (self._times_demanded[key], tick) if lfu else (tick,)
-            group = groups.get((id(target), rank))
-            if group is None:
-                group = groups[(id(target), rank)] = (target, rank, [])
-            group[2].append(key)
+            target = kept if key in protected or key in hinted else unprotected
+            tick = last_get(key, 0)
+            here = (target is kept, self._times_demanded[key], tick) if lfu else (target is kept, tick)
+            if here != at:
+                at = here
+                group = groups.get(here)
+                if group is None:
+                    group = groups[here] = (target, here[1:], [])
+                members = group[2]
+            members.append(key)
             ranked[key] = target
         for target, rank, members in groups.values():
             target.put_new(members, rank)
@@ -633,7 +661,8 @@ class ExpertCache:
             raise CacheError("only a true routing reveals demand")
         if not isinstance(token_counts, Mapping):
             raise CacheError("token counts must be a mapping expert -> tokens")
-        counts = tuple(sorted(dict(token_counts).items(), key=_order_item))
+        given = dict(token_counts)
+        counts = tuple([(key, given[key]) for key in sorted(given, key=_fields)])
         if not counts:
             raise CacheError("an empty demand cannot be revealed")
         registry, layer = self.expert_bytes, identity.layer
@@ -690,11 +719,17 @@ class ExpertCache:
         self._reveal = _Reveal(identity, counts, valid, observations, set(physical))
         # open experts cannot be evicted: they leave the rankings (what
         # _reindex does for a key that is not evictable)
-        ranked = self._ranked
+        ranked, leaving = self._ranked, {}
         for key in physical:
             home = ranked.pop(key, None)
             if home is not None:
-                home.discard(key)
+                group = leaving.get(id(home))
+                if group is None:
+                    leaving[id(home)] = (home, [key])
+                else:
+                    group[1].append(key)
+        for home, keys in leaving.values():
+            home.discard_many(keys)
         return observations
 
     def _observe(self, key, tokens, valid_tokens):
@@ -720,33 +755,38 @@ class ExpertCache:
         n = self._counters
         n["physical_layer_events"] += 1
         n["demand_events"] += int(any(o[2] for o in observations))
-        demanded, last_tick = self._times_demanded, self._last_tick
-        tokens = padding = ready = 0
-        pad_only = demands = d_tokens = d_bytes = 0
-        hits = hit_tokens = hit_bytes = 0
-        kinds = {}
-        for key, t, valid, nbytes, state, pool, source in observations:
-            tokens += t
-            padding += t - valid
-            hit = source is not None
-            ready += hit
-            if not valid:
-                pad_only += 1
-                continue
-            demanded[key] += 1
-            last_tick[key] = tick
-            demands += 1
-            d_tokens += valid
-            d_bytes += nbytes
-            if hit:
-                hits += 1
-                hit_tokens += valid
-                hit_bytes += nbytes
-                for name in (_HIT_KIND[source], "cache_resident_hits" if pool == "cache" else "staging_ready_hits"):
-                    kinds[name] = kinds.get(name, 0) + 1
+        # whole columns at a time (sums, counts and the per-key maps in C)
+        _, t_all, v_all, _, _, _, source_all = zip(*observations)
+        tokens, valid_tokens = sum(t_all), sum(v_all)
+        padding, ready = tokens - valid_tokens, len(source_all) - source_all.count(None)
+        counted = observations if 0 not in v_all else [o for o in observations if o[2]]
+        pad_only, demands = len(observations) - len(counted), len(counted)
+        d_bytes = hits = hit_tokens = hit_bytes = 0
+        pairs = {}   # (source, pool) of a hit or (None, state) of a miss -> observations
+        if counted:
+            keys, _, valids, sizes, states, pools, sources = zip(*counted)
+            self._times_demanded.update(keys)
+            self._last_tick.update(dict.fromkeys(keys, tick))
+            d_bytes = sum(sizes)
+            misses = sources.count(None)
+            if not misses:
+                hits, hit_tokens, hit_bytes = demands, valid_tokens, d_bytes
+                pairs = Counter(zip(sources, pools))
             else:
-                name = "loading_misses" if state in ("loading", "in_use") else "absent_misses"
-                kinds[name] = kinds.get(name, 0) + 1
+                hits = demands - misses
+                hit_tokens = sum([v for v, source in zip(valids, sources) if source is not None])
+                hit_bytes = sum([size for size, source in zip(sizes, sources) if source is not None])
+                pairs = Counter([(source, state if source is None else pool)
+                                 for source, pool, state in zip(sources, pools, states)])
+        d_tokens = valid_tokens
+        kinds = {}
+        for (source, at), v in pairs.items():
+            if source is not None:
+                names = _HIT_KIND[source], "cache_resident_hits" if at == "cache" else "staging_ready_hits"
+            else:
+                names = ("loading_misses" if at in ("loading", "in_use") else "absent_misses",)
+            for name in names:
+                kinds[name] = kinds.get(name, 0) + v
         n["physical_expert_demands"] += len(observations)
         n["physical_demand_tokens"] += tokens
         n["padding_token_assignments"] += padding
@@ -901,6 +941,7 @@ class ExpertCache:
         transitions; a failing handle leaves the earlier ones released)."""
         r, counters, copies = self._reveal, self._counters, self._copies
         completed = []   # cache-pool experts completed here, re-ranked together
+        done = done_valid = 0
         try:
             for handle in handles:
                 ticket = handle.ticket
@@ -917,13 +958,16 @@ class ExpertCache:
                 if holders:
                     continue
                 r.open_keys.discard(key)
-                counters["gpu_completed_experts"] += 1
-                counters["gpu_completed_valid_experts"] += int(valid)
+                done += 1
+                done_valid += valid
                 if c.ticket.pool == "demand_staging":
                     self._drop(key)
                 else:
                     completed.append(key)
         finally:
+            if done:
+                counters["gpu_completed_experts"] += done
+                counters["gpu_completed_valid_experts"] += done_valid
             if completed:
                 self._reindex_many(completed)
 

@@ -520,8 +520,9 @@ class PDScopeCudaRuntime:
             # in expert order): all resident, none loading, no demand
             decision = None
             cpu_list, demand = [], []
+            # (most tokens first, then by id: counts lists the ids in order)
             resident = ([o[0].expert for o in observations] if T == 1
-                        else sorted(counts, key=lambda e: (-counts[e], e)))
+                        else sorted(counts, key=counts.__getitem__, reverse=True))
         elif planned:
             views = {e: self.cache.residency(key(e)) for e in counts}
             hit_rate = observed["hits"] / observed["total"] if observed["total"] else 0.0
