@@ -175,6 +175,9 @@ int pdscope_grouped_block_m(int rows_hint);
  * often, which costs more than it saves once a few experts span several
  * row tiles (skewed routing). */
 int pdscope_grouped_block_m_max(int mean_rows, int max_rows);
+/* pdscope_grouped_block_m for nsel experts of intermediate I (all of them
+ * expected to be touched): 64 instead of 32 where that fills the device better. */
+int pdscope_grouped_block_m_shape(int rows_hint, int nsel, int I);
 
 /*
  * A4 grouped SwiGLU for prefill: replaces expert_forward

@@ -631,6 +631,14 @@ static int grouped_check(int phase, int block_m, const GroupedArgs &a) {
     return kOk;
 }
 
+// Whether `tiles` equal tiles on `slots` workgroups end in a round that fills
+// at most half of them, early enough (below four rounds) to cost a good part
+// of the launch.
+static bool sparse_last_round(int tiles, int slots) {
+    const int rest = tiles % slots;
+    return tiles > slots && tiles < 4 * slots && rest != 0 && 2 * rest <= slots;
+}
+
 static int grouped_phase(int phase, int block_m, const GroupedArgs &a) {
     int rc = grouped_check(phase, block_m, a);
     if (rc != kOk) return rc;
@@ -647,8 +655,18 @@ static int grouped_phase(int phase, int block_m, const GroupedArgs &a) {
         // gate/up: split load roles, 3 + 4 stages, one workgroup per CU; down
         // (K = I, a short K loop): every wave loads both operands, 2 + 2
         // stages, two workgroups per CU (T=512: 79.6 against 85.3 us)
-        if (phase & 1) rc = launch_grouped<64, 256, 64, 2, 4, 3, 4, false, 1>(1, a);
-        if (rc == kOk && (phase & 2)) rc = launch_grouped<64, 256, 64, 2, 4, 2, 2, false, 2, 2>(2, a);
+        // Half-width tiles, two workgroups per CU, where one m-tile per expert of
+        // the full width ends in a sparse round on 256 CUs (96 experts of I = 384
+        // are 288 tiles: T=201 52 -> 45 us, T=450 54 -> 47; H = 1536 down 27 ->
+        // 25).  With full rounds they read alike (T=512 Qwen shape 133.4 against
+        // 133.8) or slower (DeepSeek-V2-Lite shape T=300 125 against 127).
+        if (a.H % 256) return fail(kEInval, "grouped: H must divide by 256");
+        if (phase & 1)
+            rc = sparse_last_round(a.nsel * (a.I / 128), 256) ? launch_grouped<64, 128, 64, 2, 2, 3, 3, false, 1, 2>(1, a)
+                                                              : launch_grouped<64, 256, 64, 2, 4, 3, 4, false, 1>(1, a);
+        if (rc == kOk && (phase & 2))
+            rc = sparse_last_round(a.nsel * (a.H / 256), 512) ? launch_grouped<64, 128, 64, 2, 2, 3, 3, false, 2, 2>(2, a)
+                                                              : launch_grouped<64, 256, 64, 2, 4, 2, 2, false, 2, 2>(2, a);
         return rc;
     case 128:
         return launch_grouped<128, 256, 64, 2, 4, 3, 3>(phase, a);
@@ -702,6 +720,14 @@ PD_API int pdscope_grouped_block_m(int rows_hint) {
     // activation rows fewer times
     if (rows_hint <= 320) return 384;
     return 256;
+}
+
+// The row tile for a mean of rows_hint rows over nsel experts of intermediate
+// I: pdscope_grouped_block_m, except that thin experts take the 64-row tile
+// where its half-width form fills the chip better (see block_m 64 above).
+PD_API int pdscope_grouped_block_m_shape(int rows_hint, int nsel, int I) {
+    const int bm = pdscope_grouped_block_m(rows_hint);
+    return bm == 32 && rows_hint >= 1 && sparse_last_round(nsel * (I / 128), 256) ? 64 : bm;
 }
 
 PD_API int pdscope_grouped_block_m_max(int mean_rows, int max_rows) {

@@ -160,7 +160,7 @@ def experts_resident(x, ids, weights, slots, ws: MoEWorkspace, out=None, *, bloc
         ops.swiglu_decode(x, ids, weights, slots, H, I, ws.h_ws, out, merge=merge)
         return out
     _, _, _, packed = ws.views(T)
-    bm = block_m or ops.grouped_block_m((T * k) // E)
+    bm = block_m or ops.grouped_block_m_shape((T * k) // E, E, I)
     bmd = down_block_m(bm, H, I)
     # the balanced schedule of all experts comes out of the pack launch
     sched = (ws.sel_all, bm, ws.sel_order, ws.tile_start) + ((bmd, ws.tile_start_down) if bmd != bm else ())

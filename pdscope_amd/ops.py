@@ -207,6 +207,11 @@ def grouped_block_m(rows_hint: int, max_rows: int | None = None) -> int:
     return int(_lib.load().pdscope_grouped_block_m_max(int(rows_hint), int(max_rows)))
 
 
+def grouped_block_m_shape(rows_hint: int, nsel: int, I: int) -> int:
+    """Row tile for rows_hint mean rows over nsel experts of intermediate I."""
+    return int(_lib.load().pdscope_grouped_block_m_shape(int(rows_hint), int(nsel), int(I)))
+
+
 def schedule(counts, sel, block_m, out=None, order=None, *, block_m2=None, out2=None):
     """Tile prefix over `sel` (order=None), or, with an int32 [nsel] `order`
     buffer, the balanced order of pdscope_schedule_balanced and the prefix

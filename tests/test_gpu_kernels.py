@@ -623,6 +623,28 @@ def test_deepseek_v2_lite_layer_with_shared_experts(orc, pd):
     assert m["max_rel"] <= MAX_REL and m["mean_abs"] <= MEAN_ABS, m
 
 
+def test_half_width_tiles_equal_the_full_width_ones(pd):
+    """96 experts of I = 384 and H = 1536 leave the last round of full-width
+    64-row tiles sparse, so the 64-row launches take half-width tiles: the bits
+    are those of the 128-row launches; fewer experts keep the full width."""
+    ops, layer, synthetic = pd
+    H, I, E, k, T = 1536, 384, 96, 6, 300
+    assert ops.grouped_block_m_shape(12, E, I) == 64 and ops.grouped_block_m_shape(12, 64, I) == 32
+    assert ops.grouped_block_m_shape(12, 128, 768) == 32 and ops.grouped_block_m_shape(0, E, I) == 32
+    lay = synthetic.make_layer(H, I, E, k, True, seed=4, device=DEV)
+    x = synthetic.make_tokens(T, H, seed=5, device=DEV)
+    bias = synthetic.zipf_bias(E, 1.1, seed=6, device=DEV)[0]
+    slots = ops.slot_table([lay.experts[e] for e in range(E)], DEV)
+    outs = []
+    for bm in (64, 128):
+        ws = layer.MoEWorkspace(T, H, I, E, k, DEV)
+        out, *_ = layer.moe_forward(x, lay.gate, slots, ws, bias=bias, block_m=bm)
+        torch.cuda.synchronize()
+        outs.append((out.clone(), ws.y[:T * k * H].clone(), ws.h_ws[:T * k * I].clone()))
+    for a, b in zip(*outs):
+        assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("T,bm,bmd,skew", [(1, 32, 32, False), (33, 32, 32, True), (65, 64, 64, False),
                                            (129, 128, 128, True), (255, 256, 256, False), (257, 384, 256, False),
                                            (700, 384, 256, True), (385, 384, 384, False)])
