@@ -17,11 +17,20 @@ BF16 = torch.bfloat16
 
 
 def _p(t):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    """Device address for a c_void_p argument (None: null)."""
+    return None if t is None else t.data_ptr()
 
 
-def _stream(device) -> ctypes.c_void_p:
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
+def _stream(device) -> int:
+    """Raw handle of the current stream on `device` (a tensor's device, so with
+    an index).  Asked from torch directly: building the Stream object of
+    torch.cuda.current_stream costs about 3 us, and a layer asks four times."""
+    if _raw_stream is not None and device.index is not None:
+        return _raw_stream(device.index)
+    return torch.cuda.current_stream(device).cuda_stream
 
 
 def _need(t, name, dtype=None, ndim=None, device=None):
