@@ -34,11 +34,13 @@ __device__ __forceinline__ uint64_t group_mask(int e, bool valid) {
 // inclusive scan of one value per thread over the first 256 threads
 __device__ int block_scan256(int v, int *s_wsum) {
     const int lane = lane_id(), wave = threadIdx.x >> 6;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-        int o = __shfl_up(v, off, kWave);
-        if (lane >= off) v += o;
-    }
+    // wave scan by lane moves (a shuffle scan is six LDS round trips)
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);  // row_shr:1
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);  // row_shr:2
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);  // row_shr:4
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);  // row_shr:8
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // row_bcast:15 into rows 1, 3
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // row_bcast:31 into rows 2, 3
     if (lane == 63 && wave < 4) s_wsum[wave] = v;
     __syncthreads();
     int add = 0;
@@ -51,28 +53,37 @@ __device__ int block_scan256(int v, int *s_wsum) {
 // calling block (every thread of the block must call it: it synchronises).
 // rows[e]: rows of expert e < E (global or LDS); a sel entry outside [0, E)
 // counts as an expert with no rows (no tiles: the grouped launch never
-// addresses it).  s_rows / s_at: 256 ints of LDS each (s_rows 16-byte
-// aligned), s_wsum: 4 ints.
+// addresses it).  s_key / s_at / s_rows: 256 words of LDS each (s_key 16-byte
+// aligned), s_wsum: 4 ints.  Bound by latency on one workgroup: ranks are
+// counted over unique keys (rows, then earlier position first: one compare per
+// entry), and a rank carries its expert and rows to its place, so nothing is
+// read from memory a second time.  Pack launch with the schedule of 128
+// experts: 32 ids 6.8 -> 4.7 us, 1608 ids 8.3 -> 5.4 (64 experts took 4.7 before);
+// scatter of 32768 ids 10.9 -> 7.8 with the histogram loads unrolled.
 __device__ void balanced_schedule(const int32_t *rows, int E, const int32_t *__restrict__ sel, int nsel, int bm,
                                   int32_t *__restrict__ order, int32_t *__restrict__ tile_start, int bm2,
-                                  int32_t *__restrict__ tile_start2, int *s_rows, int *s_at, int *s_wsum) {
+                                  int32_t *__restrict__ tile_start2, uint64_t *s_key, int *s_at, int *s_rows,
+                                  int *s_wsum) {
     const int i = threadIdx.x;
+    int e = -1, c = 0;
     if (i < 256) {
-        const int e = i < nsel ? sel[i] : -1;
-        // -1 past nsel: never ranks above a real expert
-        s_rows[i] = i < nsel ? ((unsigned)e < (unsigned)E ? rows[e] : 0) : -1;
+        if (i < nsel) {
+            e = sel[i];
+            c = (unsigned)e < (unsigned)E ? rows[e] : 0;
+        }
+        // 0 past nsel: never ranks above a real expert
+        s_key[i] = i < nsel ? ((uint64_t)(uint32_t)c << 32) | (uint32_t)(256 - i) : 0;
     }
     __syncthreads();
     if (i < nsel) {
-        const int c = s_rows[i];
+        const uint64_t mine = s_key[i];
         int r = 0;
-        // four rows per LDS read (broadcast)
-        for (int j = 0; j < nsel; j += 4) {
-            const int4 q = *reinterpret_cast<const int4 *>(s_rows + j);
-            r += (q.x > c) | ((q.x == c) & (j < i));
-            r += (q.y > c) | ((q.y == c) & (j + 1 < i));
-            r += (q.z > c) | ((q.z == c) & (j + 2 < i));
-            r += (q.w > c) | ((q.w == c) & (j + 3 < i));
+        // two keys per LDS read (broadcast), several reads in flight
+#pragma unroll 8
+        for (int j = 0; j < nsel; j += 2) {
+            const ulonglong2 q = *reinterpret_cast<const ulonglong2 *>(s_key + j);
+            r += (uint64_t)q.x > mine;
+            r += (uint64_t)q.y > mine;
         }
         const int full = nsel >> 3, rem = nsel & 7;
         const int rd = r >> 3, w = r & 7;
@@ -81,15 +92,15 @@ __device__ void balanced_schedule(const int32_t *rows, int E, const int32_t *__r
         // round reaches them (round `full` deals to 0.. upward when even, 7.. downward when odd)
         int before = g * full;
         if (rem) before += (full & 1) ? max(0, g - (8 - rem)) : min(g, rem);
-        s_at[before + rd] = i;
+        s_at[before + rd] = e;
+        s_rows[before + rd] = c;
     }
     __syncthreads();
     int tiles = 0, tiles2 = 0;
     if (i < nsel) {
-        const int si = s_at[i];
-        order[i] = sel[si];
-        tiles = (s_rows[si] + bm - 1) / bm;
-        if (tile_start2) tiles2 = (s_rows[si] + bm2 - 1) / bm2;
+        order[i] = s_at[i];
+        tiles = (s_rows[i] + bm - 1) / bm;
+        if (tile_start2) tiles2 = (s_rows[i] + bm2 - 1) / bm2;
     }
     const int incl = block_scan256(tiles, s_wsum);
     if (i == 0) tile_start[0] = 0;
@@ -139,13 +150,14 @@ struct PackSchedule {
 // The schedule from the per-expert totals `tot` held by threads e < E.
 __device__ void pack_then_schedule(const PackSchedule &ps, int E, int tot) {
     __shared__ __align__(16) int s_tot[kPackMaxE];
-    __shared__ __align__(16) int s_rows[256];
+    __shared__ __align__(16) uint64_t s_key[256];
+    __shared__ int s_rows[256];
     __shared__ int s_at[256];
     __shared__ int s_ws2[4];
     if (threadIdx.x < E) s_tot[threadIdx.x] = tot;
     __syncthreads();
-    balanced_schedule(s_tot, E, ps.sel, ps.nsel, ps.bm, ps.order, ps.tile_start, ps.bm2, ps.tile_start2, s_rows,
-                      s_at, s_ws2);
+    balanced_schedule(s_tot, E, ps.sel, ps.nsel, ps.bm, ps.order, ps.tile_start, ps.bm2, ps.tile_start2, s_key,
+                      s_at, s_rows, s_ws2);
 }
 
 __global__ __launch_bounds__(1024) void pack_kernel(const int32_t *__restrict__ ids, int T, int k, int E,
@@ -298,6 +310,7 @@ __global__ __launch_bounds__(1024) void pack_scatter_kernel(const int32_t *__res
         // per-chunk counts, then the schedule, beside the scatter
         int tot = 0;
         if (threadIdx.x < E)
+#pragma unroll 8
             for (int b = 0; b < nchunk; ++b) tot += hist[(size_t)b * E + threadIdx.x];
         pack_then_schedule(ps, E, tot);
         return;
@@ -313,6 +326,7 @@ __global__ __launch_bounds__(1024) void pack_scatter_kernel(const int32_t *__res
     int tot = 0, pre = 0;
     if (threadIdx.x < E) {
         const int e = threadIdx.x;
+#pragma unroll 8
         for (int b = 0; b < nchunk; ++b) {
             const int c = hist[(size_t)b * E + e];
             tot += c;
@@ -392,10 +406,11 @@ __global__ __launch_bounds__(256) void schedule_balanced_kernel(const int32_t *_
                                                                 int32_t *__restrict__ order,
                                                                 int32_t *__restrict__ tile_start, int bm2,
                                                                 int32_t *__restrict__ tile_start2) {
-    __shared__ __align__(16) int s_rows[256];
-    __shared__ int s_at[256];  // list position -> sel position
+    __shared__ __align__(16) uint64_t s_key[256];
+    __shared__ int s_rows[256];
+    __shared__ int s_at[256];
     __shared__ int s_wsum[4];
-    balanced_schedule(counts, E, sel, nsel, bm, order, tile_start, bm2, tile_start2, s_rows, s_at, s_wsum);
+    balanced_schedule(counts, E, sel, nsel, bm, order, tile_start, bm2, tile_start2, s_key, s_at, s_rows, s_wsum);
 }
 
 }  // namespace pd

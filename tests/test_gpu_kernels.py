@@ -180,6 +180,33 @@ def test_pack_uniform(orc, pd, T, k, E):
     _pack_check(orc, ops, ids, E)
 
 
+@pytest.mark.parametrize("nsel", [1, 2, 63, 64, 65, 127, 255, 256])
+def test_balanced_schedule_ranks(pd, nsel):
+    """The balanced order over equal, zero and distinct row counts and sel
+    entries outside the experts: ranks by rows, equal rows by position, dealt
+    to eight groups in snake order; tile prefixes over that order."""
+    ops, _, _ = pd
+    rng = np.random.default_rng(nsel)
+    E = 256
+    for hi in (1, 3, 1000):
+        counts = rng.integers(0, hi, E).astype(np.int32)
+        sel = rng.permutation(E)[:nsel].astype(np.int32)
+        if nsel > 2:
+            sel[rng.integers(nsel)] = -1
+            sel[rng.integers(nsel)] = E
+        rows = [int(counts[e]) if 0 <= e < E else 0 for e in sel]
+        rank = sorted(range(nsel), key=lambda i: (-rows[i], i))
+        groups = [[] for _ in range(8)]
+        for r, i in enumerate(rank):
+            groups[r % 8 if (r // 8) % 2 == 0 else 7 - r % 8].append(i)
+        want = [i for g in groups for i in g]
+        order = torch.empty(nsel, dtype=torch.int32, device=DEV)
+        ts = ops.schedule(torch.from_numpy(counts).to(DEV), torch.from_numpy(sel).to(DEV), 32, order=order)
+        torch.cuda.synchronize()
+        assert order.cpu().tolist() == [int(sel[i]) for i in want]
+        assert ts.cpu().tolist() == [0] + np.cumsum([(rows[i] + 31) // 32 for i in want]).tolist()
+
+
 def test_pack_zipf_skew(orc, pd):
     ops, _, _ = pd
     rng = np.random.default_rng(5)
