@@ -2,10 +2,10 @@
 
 ``moe_forward`` is the whole GPU layer for experts addressed through a slot
 table: route (K1) -> decode GEMV (K4) for T == 1 (with or without shared
-experts), or pack (K2) -> balanced tile
-schedule -> grouped SwiGLU (K3) -> merge (K5) for T > 1.  Nothing is
-allocated and nothing is read back to the host, so the call can be captured
-in a hipGraph (torch.cuda.CUDAGraph) and replayed.
+experts), or pack (K2) -> balanced tile schedule -> grouped SwiGLU (K3, with
+the shared experts' tiles) -> merge (K5) for T > 1.  Nothing is allocated and
+nothing is read back to the host, so the call can be captured in a hipGraph
+(torch.cuda.CUDAGraph) and replayed.
 """
 from __future__ import annotations
 
