@@ -216,7 +216,8 @@ int pdscope_swiglu_grouped_down(const void *h_ws, const int32_t *offsets, const 
  * always-on shared experts as further tiles of the same two launches:
  * h_shared [T, shared_I] and y_shared [T, H] bf16 receive the MLP
  * shared_slot[0] (gate|up|down block of intermediate shared_I) over rows
- * 0 .. T-1 of x (shared_slot NULL: none).  With block_m == 384 and
+ * 0 .. T-1 of x (shared_slot NULL: none; an entry without a copy, NULL, gives
+ * y_shared = 0).  With block_m == 384 and
  * block_m_down == 256 the gate/up launch takes whichever of the two row tiles
  * suits the rows (chosen on the device; H % 256 == 0, I % 128 == 0).
  */

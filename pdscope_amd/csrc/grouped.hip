@@ -216,9 +216,17 @@ __device__ __forceinline__ void grouped_tile(
     }
     const int K = GATEUP ? H : I;
     const int n0 = nt * (GATEUP ? BN / 2 : BN);  // first intermediate (gate/up) or output column
-    if (base == nullptr) return;  // no ready copy of this expert: never dereference
-    const size_t IH = (size_t)I * H;
     uint16_t *const out = shared ? (GATEUP ? sh.h : sh.y) : out_routed;
+    if (base == nullptr) {
+        // no ready copy: never dereferenced.  Routed rows keep what y holds
+        // (another launch may have written them); y of the shared experts is
+        // added to every token, so without a copy it is zero
+        if (shared && !GATEUP)
+            for (int c = threadIdx.x; c < min(BM, row_end - m0) * (BN / 8); c += 64 * NW)
+                st_through(out + (size_t)(m0 + c / (BN / 8)) * H + n0 + c % (BN / 8) * 8, make_uint4(0, 0, 0, 0));
+        return;
+    }
+    const size_t IH = (size_t)I * H;
 
     // ---- per-lane source rows: load q of A-wave wa covers A rows
     // RPI(wa + NWA q) .. +RPI-1 (B likewise with wb, NWB); lane l takes row

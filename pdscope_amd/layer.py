@@ -50,11 +50,9 @@ class MoEWorkspace:
         if shared_I:
             self.h_shared = torch.empty(max_tokens * shared_I, dtype=BF16, device=device)
             self.y_shared = torch.empty((max_tokens, H), dtype=BF16, device=device)
-            self.shared_rows = torch.arange(max_tokens, **i32)
-            self.shared_offsets = torch.zeros(2, **i32)
-            self.shared_tiles = torch.zeros(2, **i32)
+            # tables of a launch without routed experts (shared_forward)
             self.shared_sel = torch.zeros(1, **i32)
-            self._shared_key = None    # (T, row tile) the two tables above hold
+            self.shared_tiles = torch.zeros(2, **i32)
             self._side = None
 
     def side_stream(self):
@@ -129,18 +127,14 @@ def shared_block_m(T: int, I: int) -> int:
 def shared_forward(x, shared_slot, ws: MoEWorkspace):
     """Always-on shared experts (DeepSeek-V2 `shared_experts`, one MLP of
     intermediate ws.shared_I applied to every token, unweighted): the grouped
-    SwiGLU kernel with a single 'expert' whose rows are all T tokens in order.
-    shared_slot: int64 [1] device table holding the shared gate|up|down block.
-    Returns y_shared [T, H] bf16."""
+    launches with shared tiles and no routed ones.
+    shared_slot: int64 [1] device table holding the shared gate|up|down block
+    (a null entry gives zeros).  Returns y_shared [T, H] bf16."""
     T = x.shape[0]
-    H, Is = ws.H, ws.shared_I
+    H, Is, sel, tiles = ws.H, ws.shared_I, ws.shared_sel, ws.shared_tiles
     bm = shared_block_m(T, Is)
-    if ws._shared_key != (T, bm):   # the one-expert tables depend only on T and the row tile
-        ws.shared_offsets[1:].fill_(T)
-        ws.shared_tiles[1:].fill_((T + bm - 1) // bm)
-        ws._shared_key = (T, bm)
-    ops.swiglu_grouped(x, ws.shared_rows[:T], ws.shared_offsets, ws.shared_sel, ws.shared_tiles,
-                       (T + bm - 1) // bm, bm, shared_slot, H, Is, ws.h_shared, ws.y_shared)
+    ops.swiglu_grouped_layer(x, sel, tiles, sel, tiles, 1, bm, tiles, 1, bm, shared_slot, H, Is, ws.h_shared,
+                             ws.y_shared, shared=(shared_slot, Is, ws.h_shared, ws.y_shared))
     return ws.y_shared[:T]
 
 

@@ -674,3 +674,28 @@ def test_one_token_with_shared_experts_without_copies(pd):
         assert bool((out == 0).all()) == (shared is none)
     assert not layer.decode_shared_fits(layer.MoEWorkspace(1, 512, 256, 32, 9, DEV, shared_I=Is))
     assert not layer.decode_shared_fits(layer.MoEWorkspace(1, 512, 192, 32, 4, DEV, shared_I=Is))
+
+
+@pytest.mark.parametrize("Is", [256, 192])   # tiles of the routed launches; launches of their own
+@pytest.mark.parametrize("T", [1, 2, 33, 300])
+def test_an_empty_shared_entry_adds_nothing(pd, T, Is):
+    """A shared table entry without a copy (null) contributes zero at every
+    token count, whatever the workspace's buffers held before the call."""
+    ops, layer, synthetic = pd
+    H, I, E, k = 512, 256, 32, 4
+    lay = synthetic.make_layer(H, I, E, k, True, seed=5, device=DEV, shared_I=Is)
+    x = synthetic.make_tokens(T, H, seed=6, device=DEV)
+    slots = ops.slot_table([lay.experts[e] for e in range(E)], DEV)
+    none = torch.zeros(1, dtype=torch.int64, device=DEV)
+    ws = layer.MoEWorkspace(T, H, I, E, k, DEV, shared_I=Is)
+    assert layer.shared_in_grouped(ws) is (Is == 256)
+    ws.y_shared.fill_(7.0)
+    ws.h_shared.fill_(7.0)
+    out, *_ = layer.moe_forward(x, lay.gate, slots, ws, shared_slot=none)
+    torch.cuda.synchronize()
+    assert bool((ws.y_shared == 0).all())
+    if T > 1:   # one token without shared experts runs on another kernel
+        plain = layer.MoEWorkspace(T, H, I, E, k, DEV)
+        ref, *_ = layer.moe_forward(x, lay.gate, slots, plain)
+        torch.cuda.synchronize()
+        assert torch.equal(out, ref)
