@@ -190,9 +190,9 @@ int pdscope_grouped_block_m_shape(int rows_hint, int nsel, int I);
  *   y[r] = bf16(h[r] . down_e^T)                      (y [T*k, H] bf16)
  * bf16 MFMA with fp32 accumulation.  max_tiles bounds sum ceil(m_e/block_m)
  * (e.g. ceil(rows/block_m) + nsel); tiles beyond tile_start[nsel] exit.
- * block_m: 32, 64, 128 or 256, the row tile pdscope_schedule used.
- * Limits: H % 256 == 0 and I % 128 == 0 (every row tile is 256 columns
- * wide: 128 gate + 128 up columns, or 256 output columns).
+ * block_m: 32, 64, 128, 256 or 384, the row tile pdscope_schedule used.
+ * Limits: H % 256 == 0 and I % 128 == 0 (256 columns: 128 gate + 128 up, or
+ * 256 output); block_m 384 (half as wide): H % 128 == 0 and I % 64 == 0.
  */
 int pdscope_swiglu_grouped(const void *x, const int32_t *perm_token, const int32_t *offsets,
                            const int32_t *sel, int nsel, const int32_t *tile_start,

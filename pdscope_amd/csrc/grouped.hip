@@ -605,10 +605,7 @@ static unsigned grouped_grid(const GroupedArgs &a, int max_tiles, int BM, int nt
 template <int BM, int BN, int BK, int WM, int WN, int SA, int SB, bool ILV = false, int PH = 3, int OCC = 1,
           int FK = 32>
 int launch_grouped(int phase, const GroupedArgs &a) {
-    if (a.I % (BN / 2) || a.H % BN || a.H % BK || a.I % BK)
-        return fail(kEInval, "grouped: I must divide by BN/2, H by BN, and both by the K step");
-    if (a.sh.slot && (a.sh.I % (BN / 2) || a.sh.I % BK))
-        return fail(kEInval, "grouped: the shared I must divide by BN/2 and the K step");
+    static_assert(BK == 64, "grouped_check: H and I divide by 64");
     if constexpr ((PH & 1) != 0) if (phase & 1) {
         grouped_kernel<BM, BN, BK, WM, WN, SA, SB, ILV, true, OCC, FK>
             <<<grouped_grid(a, a.max_tiles, BM, a.I / (BN / 2), a.sh.I / (BN / 2)), 64 * WM * WN, 0, a.s>>>(
@@ -625,17 +622,22 @@ int launch_grouped(int phase, const GroupedArgs &a) {
     return kOk;
 }
 
+// Every check of a call, before anything is launched.  A row tile of 384 takes
+// 128 columns, the others 256 (also where a narrower form of the tile runs:
+// which shapes are taken does not depend on the number of experts).
 static int grouped_check(int phase, int block_m, const GroupedArgs &a) {
     if (((phase & 1) && (!a.x || !a.perm_token)) || !a.offsets || !a.sel || !a.tile_start || !a.slots || !a.h_ws ||
         ((phase & 2) && !a.y))
         return fail(kEInval, "grouped: null pointer");
     if (a.nsel < 1 || a.max_tiles < 1) return fail(kEInval, "grouped: need nsel >= 1 and max_tiles >= 1");
-    if (a.H % 64 || a.I % 64 || a.H < 64 || a.I < 64)
-        return fail(kEInval, "grouped: need H % 64 == 0 and I % 64 == 0");
     if (a.max_tiles > (1 << 22)) return fail(kEInval, "grouped: max_tiles too large");
-    if (a.sh.slot && (a.sh.I < 64 || a.sh.T < 1 || !a.sh.h || !a.sh.y))
-        return fail(kEInval, "grouped: bad shared arguments");
-    if (block_m == 32 && a.H % 256) return fail(kEInval, "grouped: H must divide by 256");
+    if (block_m != 32 && block_m != 64 && block_m != 128 && block_m != 256 && block_m != 384)
+        return fail(kEInval, "grouped: block_m must be 32, 64, 128, 256 or 384");
+    const int cols = block_m == 384 ? 128 : 256;
+    if (a.H < cols || a.H % cols || a.I < cols / 2 || a.I % (cols / 2))
+        return fail(kEInval, "grouped: need H % 256 == 0 and I % 128 == 0 (block_m 384: H % 128, I % 64)");
+    if (a.sh.slot && (a.sh.I < cols / 2 || a.sh.I % (cols / 2) || a.sh.T < 1 || !a.sh.h || !a.sh.y))
+        return fail(kEInval, "grouped: bad shared arguments (shared I % 128 == 0; block_m 384: % 64)");
     return kOk;
 }
 
@@ -647,9 +649,9 @@ static bool sparse_last_round(int tiles, int slots) {
     return tiles > slots && tiles < 4 * slots && rest != 0 && 2 * rest <= slots;
 }
 
+// The launches of a checked call.
 static int grouped_phase(int phase, int block_m, const GroupedArgs &a) {
-    int rc = grouped_check(phase, block_m, a);
-    if (rc != kOk) return rc;
+    int rc = kOk;
     switch (block_m) {
     case 32:
         // down (K = I, a short K loop): two workgroups of 128 columns per CU, so
@@ -668,7 +670,6 @@ static int grouped_phase(int phase, int block_m, const GroupedArgs &a) {
         // are 288 tiles: T=201 52 -> 45 us, T=450 54 -> 47; H = 1536 down 27 ->
         // 25).  With full rounds they read alike (T=512 Qwen shape 133.4 against
         // 133.8) or slower (DeepSeek-V2-Lite shape T=300 125 against 127).
-        if (a.H % 256) return fail(kEInval, "grouped: H must divide by 256");
         if (phase & 1)
             rc = sparse_last_round(a.nsel * (a.I / 128), 256) ? launch_grouped<64, 128, 64, 2, 2, 3, 3, false, 1, 2>(1, a)
                                                               : launch_grouped<64, 256, 64, 2, 4, 3, 4, false, 1>(1, a);
@@ -690,21 +691,19 @@ static int grouped_phase(int phase, int block_m, const GroupedArgs &a) {
         // rows than the tile keeps both busy (T=2048, 128 rows each: gate/up
         // 163 -> 153 us, down 96 -> 90; T=4096 Zipf down 173 -> 162)
         return launch_grouped<256, 256, 64, 2, 4, 2, 3, true, 3, 1, 16>(phase, a);
-    case 384:
+    default:  // 384
         return launch_grouped<384, 128, 64, 4, 2, 2, 4, true>(phase, a);
-    default:
-        return fail(kEInval, "grouped: block_m must be 32, 64, 128, 256 or 384");
     }
 }
 
 static int grouped_entry(int phase, const void *x, const int32_t *perm_token, const int32_t *offsets,
                          const int32_t *sel, int nsel, const int32_t *tile_start, int max_tiles, int block_m,
                          const void *const *slots, int H, int I, void *h_ws, void *y, void *stream) {
-    return grouped_phase(phase, block_m,
-                         GroupedArgs{(const uint16_t *)x, perm_token, offsets, sel, nsel, tile_start, max_tiles,
-                                     (const uint16_t *const *)slots, H, I, (uint16_t *)h_ws, (uint16_t *)y,
-                                     SharedTiles{nullptr, 0, 0, nullptr, nullptr},
-                                     reinterpret_cast<hipStream_t>(stream)});
+    const GroupedArgs a{(const uint16_t *)x, perm_token, offsets, sel, nsel, tile_start, max_tiles,
+                        (const uint16_t *const *)slots, H, I, (uint16_t *)h_ws, (uint16_t *)y,
+                        SharedTiles{nullptr, 0, 0, nullptr, nullptr}, reinterpret_cast<hipStream_t>(stream)};
+    const int rc = grouped_check(phase, block_m, a);
+    return rc != kOk ? rc : grouped_phase(phase, block_m, a);
 }
 
 }  // namespace pd
@@ -773,15 +772,13 @@ PD_API int pdscope_swiglu_grouped_layer(const void *x, const int32_t *perm_token
     GroupedArgs d = a;
     d.tile_start = tile_start_down;
     d.max_tiles = max_tiles_down;
+    int rc = grouped_check(1, block_m, a);
+    if (rc == kOk) rc = grouped_check(2, block_m_down, d);
+    if (rc != kOk) return rc;
     if (block_m != 384 || block_m_down != 256) {
-        const int rc = grouped_phase(1, block_m, a);
+        rc = grouped_phase(1, block_m, a);
         return rc != kOk ? rc : grouped_phase(2, block_m_down, d);
     }
-    int rc = grouped_check(3, 384, a);
-    if (rc == kOk) rc = grouped_check(3, 256, d);
-    if (rc != kOk) return rc;
-    if (H % 256 || I % 128 || sh.I % 128)
-        return fail(kEInval, "grouped: the tile pair needs H % 256 == 0 and I % 128 == 0");
     const unsigned grid = std::max(grouped_grid(a, max_tiles, 384, I / 64, sh.I / 64),
                                    grouped_grid(d, max_tiles_down, 256, I / 128, sh.I / 128));
     grouped_gateup_pair_kernel<<<grid, 512, 0, a.s>>>(a.x, perm_token, offsets, sel, nsel, tile_start, tile_start_down,

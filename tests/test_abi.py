@@ -61,3 +61,48 @@ def test_invalid_arguments_raise_before_any_launch():
     with pytest.raises(ValueError, match="null binding"):
         _lib.call("pdscope_decode_run", None, None, None, None, None, None, 1, None)
     _lib.load().pdscope_decode_unbind(None)   # freeing no binding is a no-op
+
+
+GROUPED_CALLS = {
+    # entry -> arguments from (nsel, bm, bm of the down half, H, I, shared I)
+    "pdscope_swiglu_grouped": lambda p, n, bm, bd, H, I, Is: [p, p, p, p, n, p, 4, bm, p, H, I, p, p, None],
+    "pdscope_swiglu_grouped_gateup": lambda p, n, bm, bd, H, I, Is: [p, p, p, p, n, p, 4, bm, p, H, I, p, None],
+    "pdscope_swiglu_grouped_down": lambda p, n, bm, bd, H, I, Is: [p, p, p, n, p, 4, bd, p, H, I, p, None],
+    "pdscope_swiglu_grouped_layer": lambda p, n, bm, bd, H, I, Is: [p, p, p, p, n, p, 4, bm, p, 4, bd, p, H, I, p, p, 3,
+                                                                    p if Is else None, Is, p, p, None],
+}
+
+
+@pytest.mark.parametrize("entry,n,bm,bd,H,I,Is", [
+    # I off the 256-column tiles' multiple, whatever the number of experts makes
+    # of the width of the 64-row tiles (300 and 700: sparse last rounds)
+    ("pdscope_swiglu_grouped", 8, 64, 64, 1536, 192, 0),
+    ("pdscope_swiglu_grouped", 300, 64, 64, 1536, 192, 0),
+    ("pdscope_swiglu_grouped", 300, 64, 64, 32768, 192, 0),
+    ("pdscope_swiglu_grouped_gateup", 300, 64, 64, 1536, 192, 0),
+    ("pdscope_swiglu_grouped_down", 700, 64, 64, 256, 192, 0),
+    ("pdscope_swiglu_grouped_down", 8, 32, 32, 512, 192, 0),
+    ("pdscope_swiglu_grouped_down", 8, 32, 32, 640, 256, 0),
+    # 384 rows (128 columns)
+    ("pdscope_swiglu_grouped", 8, 384, 384, 192, 128, 0),
+    ("pdscope_swiglu_grouped", 8, 384, 384, 256, 96, 0),
+    # a row tile that does not exist
+    ("pdscope_swiglu_grouped", 8, 48, 48, 512, 256, 0),
+    # the down half of a pair of launches: refused before the gate/up launch
+    ("pdscope_swiglu_grouped_layer", 8, 32, 48, 512, 256, 0),
+    ("pdscope_swiglu_grouped_layer", 8, 384, 64, 640, 256, 0),
+    ("pdscope_swiglu_grouped_layer", 300, 64, 64, 1536, 192, 0),
+    # shared experts off the tile
+    ("pdscope_swiglu_grouped_layer", 300, 64, 64, 1536, 128, 192),
+    ("pdscope_swiglu_grouped_layer", 8, 384, 384, 256, 128, 96),
+    ("pdscope_swiglu_grouped_layer", 8, 384, 256, 256, 128, 192),
+])
+def test_grouped_shapes_are_refused_before_any_launch(entry, n, bm, bd, H, I, Is):
+    """A shape outside the row tile's columns is an invalid argument in every
+    grouped entry point (a launch would be a HIP error here, without a device)."""
+    import ctypes
+
+    from pdscope_amd import _lib
+    memory = ctypes.create_string_buffer(64)   # non-null; refused before it is read
+    with pytest.raises(ValueError, match="grouped"):
+        _lib.call(entry, *GROUPED_CALLS[entry](ctypes.addressof(memory), n, bm, bd, H, I, Is))
