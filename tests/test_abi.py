@@ -106,3 +106,17 @@ def test_grouped_shapes_are_refused_before_any_launch(entry, n, bm, bd, H, I, Is
     memory = ctypes.create_string_buffer(64)   # non-null; refused before it is read
     with pytest.raises(ValueError, match="grouped"):
         _lib.call(entry, *GROUPED_CALLS[entry](ctypes.addressof(memory), n, bm, bd, H, I, Is))
+
+
+def test_wide_stores_in_asm_carry_their_wait_states():
+    """gfx950 reads the data registers of a vector store of more than 8 bytes
+    after the store has issued: a VALU write to them needs two wait states in
+    between.  The compiler keeps them for stores of its own and cannot see one
+    inside an asm string, so the string has to end with them."""
+    found = 0
+    for path in sorted((ROOT / "pdscope_amd" / "csrc").iterdir()):
+        for text in re.findall(r'asm\s+(?:volatile)?\s*\(\s*((?:"[^"]*"\s*)+)', path.read_text()):
+            if re.search(r"_store_(dwordx[34]|b96|b128)", text):
+                found += 1
+                assert re.search(r"_store_\w+[^;]*\\n\\ts_nop 1\"\s*$", text), (path.name, text)
+    assert found >= 1
