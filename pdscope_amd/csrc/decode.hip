@@ -91,7 +91,11 @@ struct SharedDown {
 // pairs (k <= 2 KP) and CS 16-byte chunks per lane of a shared row (0: none).
 // Every row of the wave's output column is loaded before h is staged, so the
 // launch, bound by the bytes of the down rows, pays one memory latency instead
-// of one per slot pair (two waves a SIMD cannot hide it).
+// of one per slot pair (two waves a SIMD cannot hide it).  A pair that an odd k
+// leaves half empty reads its other half's row twice, in the same loads; with
+// h read there instead (and k <= 2 on two pairs) both decode launches took
+// 9.4 us against 7.7 at k = 1, 10.3 against 8.7 at k = 2 and 18.2 against 16.9
+// at k = 7 (H 2048, I 768; one slot pair at a time 8.1, 9.1 and 20.5).
 template <int CPL, int KP, int CS>
 __global__ __launch_bounds__(256) void decode_down_kernel(const uint16_t *__restrict__ h_ws,
                                                           const int32_t *__restrict__ ids,
@@ -110,10 +114,10 @@ __global__ __launch_bounds__(256) void decode_down_kernel(const uint16_t *__rest
     bool has[KP];
 #pragma unroll
     for (int p = 0; p < KP; ++p) {
-        const int s = 2 * p + half;
-        const uint16_t *base = s < k ? slots[ids[s]] : nullptr;
+        // past the last slot: the last slot's row again, which the other half reads
+        const uint16_t *base = slots[ids[min(2 * p + half, k - 1)]];
         has[p] = base != nullptr;
-        // no slot or no ready copy: read h itself (k*I elements, in bounds) and add 0
+        // no ready copy: read h itself (k*I elements, in bounds) and add 0
         const uint4 *row = base ? reinterpret_cast<const uint4 *>(base + IH2 + (size_t)jc * I)
                                 : reinterpret_cast<const uint4 *>(h_ws);
 #pragma unroll
@@ -290,13 +294,13 @@ static int launch_decode(const void *x, const int32_t *ids, const void *w, int k
     const int dblocks = (H + 3) / 4;
     const uint16_t *hp = (const uint16_t *)h_ws, *wp = (const uint16_t *)w;
     if (down_fits(k, I, sd.I)) {
-        const int kp = k <= 4 ? 2 : k <= 6 ? 3 : 4, cs = sd.slot ? (sd.I <= 3 * 512 ? 3 : 6) : 0;
+        const int kp = k <= 2 ? 1 : k <= 4 ? 2 : k <= 6 ? 3 : 4, cs = sd.slot ? (sd.I <= 3 * 512 ? 3 : 6) : 0;
         const int cc = cpl <= 3 ? 3 : 6;
 #define PD_DN(C, P, S)                                                                                          \
     if (cc == C && kp == P && cs == S)                                                                          \
         decode_down_kernel<C, P, S><<<dblocks, 256, lds, s>>>(hp, ids, wp, sp, H, I, k, merge_mode, sd, (uint16_t *)out);
 #define PD_DNS(C, P) PD_DN(C, P, 0) PD_DN(C, P, 3) PD_DN(C, P, 6)
-        PD_DNS(3, 2) PD_DNS(3, 3) PD_DNS(3, 4) PD_DNS(6, 2) PD_DNS(6, 3) PD_DNS(6, 4)
+        PD_DNS(3, 1) PD_DNS(3, 2) PD_DNS(3, 3) PD_DNS(3, 4) PD_DNS(6, 1) PD_DNS(6, 2) PD_DNS(6, 3) PD_DNS(6, 4)
 #undef PD_DNS
 #undef PD_DN
         return check_launch("decode_down_kernel");

@@ -699,3 +699,52 @@ def test_an_empty_shared_entry_adds_nothing(pd, T, Is):
         ref, *_ = layer.moe_forward(x, lay.gate, slots, plain)
         torch.cuda.synchronize()
         assert torch.equal(out, ref)
+
+
+@pytest.mark.parametrize("I", [64, 768, 776, 1408])   # chunks a half-wave lane holds: 1, 3, 4, 6
+@pytest.mark.parametrize("k", [1, 2, 3, 4, 5, 7, 8])
+def test_decode_slot_counts(orc, pd, k, I):
+    """swiglu_decode at every number of slot pairs, odd counts (whose last half
+    pair reads the last slot's row again) and a slot without a copy: the expert
+    rows read off k = 1 calls are the oracle's within bf16 tolerance, the
+    ordered merge of those rows is bit-exact, the fp32 one within two bf16
+    roundings of the oracle's."""
+    ops, _, synthetic = pd
+    H, E = 256, 32
+    lay = synthetic.make_layer(H, I, E, 8, True, seed=I + k, device=DEV)
+    blocks = [lay.experts[e] for e in range(E)]
+    x = synthetic.make_tokens(1, H, seed=k, device=DEV)
+    rng = np.random.default_rng(k)
+    ids = rng.permutation(E)[:k].astype(np.int32)
+    w = orc.f32_to_bf16(rng.random((1, k)).astype(np.float32))
+    slots = ops.slot_table(blocks, DEV)
+    if k > 2:
+        slots[int(ids[k // 2])] = 0
+    ids_dev = torch.from_numpy(ids).view(1, k).to(DEV)
+    one = torch.ones((1, 1), dtype=torch.bfloat16, device=DEV)
+    rank = np.argsort(np.argsort(ids)).astype(np.int32)
+    y = np.empty((k, H), np.uint16)
+    h = torch.empty(k * I, dtype=torch.bfloat16, device=DEV)
+    out = torch.empty((1, H), dtype=torch.bfloat16, device=DEV)
+    n = I * H
+    for s in range(k):
+        ops.swiglu_decode(x, ids_dev[:, s:s + 1].contiguous(), one, slots, H, I, h, out)
+        torch.cuda.synchronize()
+        y[rank[s]] = u16(out)[0]
+        b = u16(blocks[ids[s]])
+        ref = orc.bf16_to_f32(orc.expert_forward(u16(x), b[:n].reshape(I, H), b[n:2 * n].reshape(I, H),
+                                                 b[2 * n:].reshape(H, I)))
+        if k > 2 and s == k // 2:
+            ref = np.zeros_like(ref)
+            assert not u16(out).any()
+        m = err_metrics(orc.bf16_to_f32(u16(out)), ref)
+        assert m["max_rel"] <= MAX_REL and m["mean_abs"] <= MEAN_ABS, m
+    for merge in ("fused", "reference"):
+        ops.swiglu_decode(x, ids_dev, torch.from_numpy(w.view(np.int16)).view(torch.bfloat16).to(DEV), slots, H, I, h,
+                          out, merge=merge)
+        torch.cuda.synchronize()
+        if merge == "reference":
+            assert np.array_equal(u16(out), orc.merge_ordered(y, rank, w))
+        else:
+            np.testing.assert_allclose(orc.bf16_to_f32(u16(out)), orc.bf16_to_f32(orc.merge(y, rank, w)),
+                                       rtol=2.0 ** -7, atol=1e-5)
