@@ -63,13 +63,15 @@ struct MergeAcc {
 
 // k <= KM: one wave per token and 64 output chunks (512 columns).  The
 // token's k row indices and weights are the same for the whole wave: lane s
-// holds slot s, the k values become scalars by lane reads, and all k rows of
-// a lane's chunk are loaded before the first is added.
+// holds slot s, the k values become scalars by lane reads, and up to eight rows
+// of a lane's chunk are loaded before the first of them is added (sixteen leave
+// room for fewer waves: T=1400, k=16, H=2048 18.9 us against 17.3, where one
+// slot at a time took 17.4).
 // Bound by the bytes of y.  ORDERED (rows in ascending grouped row, acc =
 // bf16(acc + bf16(w * y)) per row, add_in added last): each lane ranks its
 // slot against the others (k compares) and one lane push sorts them; a loop
 // over all k for each next row in every thread took 71 us at T=4096, k=8,
-// H=2048 (about 36 now, 31 for the fp32 sum), and the roundings in integer
+// H=2048, 27 now (25 for the fp32 sum), and the roundings in integer
 // arithmetic more than the loads (now the hardware's pair conversion).
 template <int KM, bool ORDERED>
 __global__ __launch_bounds__(256) void merge_kernel(const uint16_t *__restrict__ y,
@@ -105,17 +107,20 @@ __global__ __launch_bounds__(256) void merge_kernel(const uint16_t *__restrict__
             row = __builtin_amdgcn_ds_permute(dst, row);
             wb = __builtin_amdgcn_ds_permute(dst, wb);
         }
-        uint4 v[KM];
-#pragma unroll
-        for (int s = 0; s < KM; ++s)
-            if (s < k)
-                v[s] = reinterpret_cast<const uint4 *>(y + (size_t)__builtin_amdgcn_readlane(row, s) * H)[cc];
         MergeAcc<ORDERED> acc;
         if (!ORDERED && add_in) acc.set(addv);
         else acc.zero();
+#pragma unroll 1
+        for (int b = 0; b < (KM > 8 ? k : 1); b += 8) {
+            uint4 v[8];
 #pragma unroll
-        for (int s = 0; s < KM; ++s)
-            if (s < k) acc.add(bf2f((uint32_t)__builtin_amdgcn_readlane(wb, s)), v[s]);
+            for (int s = 0; s < 8; ++s)
+                if (b + s < k)
+                    v[s] = reinterpret_cast<const uint4 *>(y + (size_t)__builtin_amdgcn_readlane(row, b + s) * H)[cc];
+#pragma unroll
+            for (int s = 0; s < 8; ++s)
+                if (b + s < k) acc.add(bf2f((uint32_t)__builtin_amdgcn_readlane(wb, b + s)), v[s]);
+        }
         if (ORDERED && add_in) acc.add_last(addv);
         if (live) reinterpret_cast<uint4 *>(out + (size_t)t * H)[c] = acc.result();
     }
