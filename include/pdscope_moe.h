@@ -163,7 +163,7 @@ int pdscope_pack_schedule_balanced(const int32_t *ids, int T, int k, int E, int3
                                    int32_t *tile_start, int32_t *tile_start2, void *stream);
 
 /* Row tile (32, 64, 128, 256 or 384) for `rows_hint` average rows per
- * selected expert: <= 16 rows 32, <= 64 rows 64, <= 124 rows 128, <= 192 rows
+ * selected expert: <= 16 rows 32, <= 44 rows 64, <= 104 rows 128, <= 192 rows
  * 256, <= 320 rows 384 (one tile holds a typical expert, so its weights
  * stream once), 256 above.  No reference counterpart: the reference launches
  * one torch GEMM chain per expert (expertbench/adapters/qwen.py:87-90). */
@@ -175,8 +175,8 @@ int pdscope_grouped_block_m(int rows_hint);
  * often, which costs more than it saves once a few experts span several
  * row tiles (skewed routing). */
 int pdscope_grouped_block_m_max(int mean_rows, int max_rows);
-/* pdscope_grouped_block_m for nsel experts of intermediate I (all of them
- * expected to be touched): 64 instead of 32 where that fills the device better. */
+/* pdscope_grouped_block_m for nsel experts of intermediate I: 64 instead of 32
+ * where that fills the device better (two or more mean rows). */
 int pdscope_grouped_block_m_shape(int rows_hint, int nsel, int I);
 
 /*

@@ -55,6 +55,12 @@ typedef __attribute__((address_space(1))) const void g_void_t;
 // 145 -> 135 and 83 -> 76; T=4096 (about half the experts have two tiles)
 // 289 -> 284 and 167 -> 160; DeepSeek-V2-Lite shape T=1304 down 95 -> 82.
 // nt throughout: T=512 with Zipf routing 159 against 148, T=4096 301.
+// Streamed lines are not kept in the Infinity Cache either, so a pass whose
+// weights all fit there (256 MB) and that is repeated at once is the one that
+// loses: 16 experts of the Qwen shape, gate/up again and again, 19.8 us under
+// sc1 and 28.8 here (32.3 and 29.3 when other experts come in between; weights
+// just copied from the host 34.3 and 29.7, 4 experts); one layer of T=2 57.0
+// and 59.5, two layers in turn 65.0 and 57.3.
 // Activation tiles keep the default policy.
 constexpr int kDeviceScope = 16;
 constexpr int kStream = 2;
@@ -668,8 +674,10 @@ static int grouped_phase(int phase, int block_m, const GroupedArgs &a) {
         // Half-width tiles, two workgroups per CU, where one m-tile per expert of
         // the full width ends in a sparse round on 256 CUs (96 experts of I = 384
         // are 288 tiles: T=201 52 -> 45 us, T=450 54 -> 47; H = 1536 down 27 ->
-        // 25).  With full rounds they read alike (T=512 Qwen shape 133.4 against
-        // 133.8) or slower (DeepSeek-V2-Lite shape T=300 125 against 127).
+        // 25; 87 of the Qwen shape's experts, 32 rows each, 107 -> 99, 106 of
+        // them 116 -> 110).  With full rounds they read alike (128 of them 131
+        // against 133, down 71 against 75) or slower (DeepSeek-V2-Lite shape T=300
+        // 125 against 127).
         if (phase & 1)
             rc = sparse_last_round(a.nsel * (a.I / 128), 256) ? launch_grouped<64, 128, 64, 2, 2, 3, 3, false, 1, 2>(1, a)
                                                               : launch_grouped<64, 256, 64, 2, 4, 3, 4, false, 1>(1, a);
@@ -731,10 +739,15 @@ PD_API int pdscope_grouped_block_m(int rows_hint) {
 
 // The row tile for a mean of rows_hint rows over nsel experts of intermediate
 // I: pdscope_grouped_block_m, except that thin experts take the 64-row tile
-// where its half-width form fills the chip better (see block_m 64 above).
+// where its half-width form fills the chip better (see block_m 64 above).  That
+// counts a tile for every expert, so it needs two rows each: at a mean of one,
+// about 0.63 of them have rows (96 experts of I = 384 are 180 tiles, no second
+// round at all).  Whole layers of that shape on 32 and 64 rows: T=16 57.8 and
+// 60.2 us, T=24 64.9 and 65.3, T=32 (two rows each) 71.3 and 70.6, T=40 86.8 and
+// 80.7, T=200 93.1 and 86.5.
 PD_API int pdscope_grouped_block_m_shape(int rows_hint, int nsel, int I) {
     const int bm = pdscope_grouped_block_m(rows_hint);
-    return bm == 32 && rows_hint >= 1 && sparse_last_round(nsel * (I / 128), 256) ? 64 : bm;
+    return bm == 32 && rows_hint >= 2 && sparse_last_round(nsel * (I / 128), 256) ? 64 : bm;
 }
 
 PD_API int pdscope_grouped_block_m_max(int mean_rows, int max_rows) {

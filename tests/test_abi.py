@@ -63,6 +63,18 @@ def test_invalid_arguments_raise_before_any_launch():
     _lib.load().pdscope_decode_unbind(None)   # freeing no binding is a no-op
 
 
+@pytest.mark.parametrize("rows,nsel,I,want", [
+    (0, 96, 384, 32), (1, 96, 384, 32), (2, 96, 384, 64), (16, 96, 384, 64), (17, 96, 384, 64), (50, 96, 384, 128),
+    (12, 128, 768, 32), (2, 64, 384, 32), (2, 85, 384, 32), (2, 86, 384, 64), (2, 128, 384, 64), (2, 129, 384, 32),
+])
+def test_row_tile_of_thin_experts(rows, nsel, I, want):
+    """Thin experts take the 64-row tile where one tile per expert ends in a
+    sparse round; a mean of one row leaves a third of the experts without rows,
+    so the launch has fewer tiles than that and keeps the 32-row tile."""
+    from pdscope_amd import _lib
+    assert _lib.load().pdscope_grouped_block_m_shape(rows, nsel, I) == want
+
+
 GROUPED_CALLS = {
     # entry -> arguments from (nsel, bm, bm of the down half, H, I, shared I)
     "pdscope_swiglu_grouped": lambda p, n, bm, bd, H, I, Is: [p, p, p, p, n, p, 4, bm, p, H, I, p, p, None],
