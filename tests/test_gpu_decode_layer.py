@@ -748,3 +748,43 @@ def test_decode_slot_counts(orc, pd, k, I):
         else:
             np.testing.assert_allclose(orc.bf16_to_f32(u16(out)), orc.bf16_to_f32(orc.merge(y, rank, w)),
                                        rtol=2.0 ** -7, atol=1e-5)
+
+
+@pytest.mark.parametrize("T", [1, 2, 5, 8])
+def test_router_with_the_shared_gateup_half(orc, pd, T):
+    """pdscope_route_topk_shared: routing bitwise pdscope_route_topk's, each
+    token's shared h that of a call with this token alone, and that one the
+    oracle's within bf16 tolerance."""
+    from pdscope_amd import _lib
+    ops, _, synthetic = pd
+    H, I, E, k, Is = 512, 128, 64, 6, 203   # shared rows end inside a block of eight
+    lay = synthetic.make_layer(H, I, E, k, False, seed=3, device=DEV, shared_I=Is)
+    x = synthetic.make_tokens(T, H, seed=T, device=DEV)
+    shared = ops.slot_table([lay.shared], DEV)
+    stream = torch.cuda.current_stream().cuda_stream
+
+    def call(rows):
+        n = rows.shape[0]
+        logits = torch.empty((n, E), dtype=torch.bfloat16, device=DEV)
+        ids = torch.empty((n, k), dtype=torch.int32, device=DEV)
+        w = torch.empty((n, k), dtype=torch.bfloat16, device=DEV)
+        h = torch.full((n, Is), 7.0, dtype=torch.bfloat16, device=DEV)
+        ws = ops.new_route_workspace(n, H, E, torch.device(DEV, 0))
+        _lib.call("pdscope_route_topk_shared", rows.data_ptr(), lay.gate.data_ptr(), None, n, H, E, k, 0,
+                  logits.data_ptr(), ids.data_ptr(), w.data_ptr(), None, ws.data_ptr(), shared.data_ptr(), Is,
+                  h.data_ptr(), stream)
+        torch.cuda.synchronize()
+        return logits, ids, w, h
+
+    logits, ids, w, h = call(x)
+    rl, ri, rw, _ = ops.route_topk(x, lay.gate, k, False)
+    torch.cuda.synchronize()
+    assert torch.equal(logits, rl) and torch.equal(ids, ri) and torch.equal(w, rw)
+    sh = u16(lay.shared)
+    n = Is * H
+    for t in range(T):
+        assert torch.equal(call(x[t:t + 1].contiguous())[3][0], h[t])
+    _, ref = orc.expert_forward(u16(x), sh[:n].reshape(Is, H), sh[n:2 * n].reshape(Is, H),
+                                sh[2 * n:].reshape(H, Is), want_h=True)
+    m = err_metrics(orc.bf16_to_f32(u16(h)), orc.bf16_to_f32(ref))
+    assert m["max_rel"] <= MAX_REL and m["mean_abs"] <= MEAN_ABS, m

@@ -672,16 +672,25 @@ def test_half_width_tiles_equal_the_full_width_ones(pd):
         assert torch.equal(a, b)
 
 
-@pytest.mark.parametrize("T,bm,bmd,skew", [(1, 32, 32, False), (33, 32, 32, True), (65, 64, 64, False),
-                                           (129, 128, 128, True), (255, 256, 256, False), (257, 384, 256, False),
-                                           (700, 384, 256, True), (385, 384, 384, False)])
-def test_grouped_layer_tiles_equal_the_plain_launches(pd, T, bm, bmd, skew):
+# H, I, E, k, shared I; the second leaves the last round of full-width 64-row
+# tiles sparse in both halves (288 on 256 workgroups, 576 on 512)
+LAYER_TILES = dict(small=(256, 128, 32, 4, 384), sparse=(1536, 384, 96, 6, 384))
+
+
+# body: the row tile the device must choose for gate/up of a 384 / 256 pair
+@pytest.mark.parametrize("T,bm,bmd,skew,shape,body", [
+    (1, 32, 32, False, "small", None), (33, 32, 32, True, "small", None), (65, 64, 64, False, "small", None),
+    (129, 128, 128, True, "small", None), (255, 256, 256, False, "small", None),
+    (257, 384, 256, False, "small", 256), (700, 384, 256, True, "small", 256), (2401, 384, 256, False, "small", 384),
+    (385, 384, 384, False, "small", None), (300, 64, 64, False, "sparse", None), (65, 64, 64, True, "sparse", None)])
+def test_grouped_layer_tiles_equal_the_plain_launches(pd, T, bm, bmd, skew, shape, body):
     """swiglu_grouped_layer (a row tile per half, the 384/256 choice on the
-    device on both sides of its rule, shared experts as further tiles) gives
-    the bits of the plain launches: every row is the same arithmetic in every
-    tile.  T around the tile heights, so the shared rows end inside a tile."""
+    device on both sides of its rule, shared experts as further tiles, also of
+    half-width launches) gives the bits of the plain launches on 128-row tiles:
+    every row is the same arithmetic in every tile.  T around the tile heights,
+    so the shared rows end inside a tile."""
     ops, layer, synthetic = pd
-    H, I, E, k, Is = 256, 128, 32, 4, 384
+    H, I, E, k, Is = LAYER_TILES[shape]
     lay = synthetic.make_layer(H, I, E, k, True, seed=T, device=DEV, shared_I=Is)
     x = synthetic.make_tokens(T, H, seed=T + 1, device=DEV)
     bias = synthetic.zipf_bias(E, 1.5, seed=2, device=DEV)[0] if skew else None
@@ -701,14 +710,16 @@ def test_grouped_layer_tiles_equal_the_plain_launches(pd, T, bm, bmd, skew):
         return (torch.full((rows * inner,), 7.0, dtype=torch.bfloat16, device=DEV),
                 torch.full((rows * H,), 7.0, dtype=torch.bfloat16, device=DEV))
 
-    order, ts, mt = tiles(64)
+    order, ts, mt = tiles(128)
     ref_h, ref_y = bufs(n, I)
-    ops.swiglu_grouped(x, packed.perm_token, packed.offsets, order, ts, mt, 64, slots, H, I, ref_h, ref_y)
+    ops.swiglu_grouped(x, packed.perm_token, packed.offsets, order, ts, mt, 128, slots, H, I, ref_h, ref_y)
     one = dict(dtype=torch.int32, device=DEV)
     ref_hs, ref_ys = bufs(T, Is)
     ops.swiglu_grouped(x, torch.arange(T, **one), torch.tensor([0, T], **one), torch.zeros(1, **one),
-                       torch.tensor([0, (T + 63) // 64], **one), (T + 63) // 64, 64, shared, H, Is, ref_hs, ref_ys)
+                       torch.tensor([0, (T + 127) // 128], **one), (T + 127) // 128, 128, shared, H, Is, ref_hs, ref_ys)
     (order, ts, mt), (_, tsd, mtd) = tiles(bm), tiles(bmd)
+    if body is not None:
+        assert (4 * int(ts[-1]) <= 3 * int(tsd[-1])) is (body == 384)
     for with_shared in (False, True):
         h, y = bufs(n, I)
         hs, ys = bufs(T, Is)
