@@ -10,8 +10,9 @@
 //   H = 2048 are 4 chunks per lane), so each wave keeps 16 loads in flight.
 //   h[s,i] = bf16(bf16(silu(bf16(g))) * bf16(u))  ->  h_ws [k, I]
 // Launch 2 (down + merge): each 32-lane half-wave owns one expert row of
-//   down_s (I bf16); a wave walks the k experts in pairs for its output
-//   column j, rounds each expert's y to bf16 (the expert output dtype) and
+//   down_s (I bf16); a wave loads the rows of all k experts for its output
+//   column j, two at a time per load, rounds each expert's y to bf16 (the expert
+//   output dtype) and
 //   accumulates w_s * y_s in fp32 in slot order (merge_mode 0:
 //   out[j] = bf16(sum_s w_s * y_s[j]), one rounding), or keeps the y_s and
 //   adds them in ascending expert id in bf16 arithmetic (merge_mode 1, the

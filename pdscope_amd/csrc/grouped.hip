@@ -120,6 +120,28 @@ __device__ __forceinline__ void wait_stage(int younger) {
     }
 }
 
+// Always-on shared experts as further tiles of a grouped launch (slot ==
+// nullptr: none): one MLP of intermediate I over rows 0 .. T-1 in order, on the
+// launch's own tile shape.  Its tiles take the first blocks of the grid: the
+// down half is the longest tile of the launch (K = shared I).  As launches of
+// their own on a second stream, on 256-row tiles that read the shared block
+// fewest times, they held CUs for long while the routed launches waited at the
+// join (48 blocks for the down half at T=1304), and their time moved with how
+// the two streams met.  DeepSeek-V2-Lite layer, then and now (today's loads and
+// stores among it): T=48 233 -> 199 us, T=128 243 -> 222, T=180 248 -> 228 (six
+// 32-row tiles), T=190 244 -> 239, T=400 257 -> 256 and T=470 272 -> 260 (eight
+// 64-row tiles), T=640 272 -> 257, T=1304 324 -> 307, T=2048 390 -> 392, T=4096
+// 699 -> 697.
+struct SharedTiles {
+    const uint16_t *const *slot;  // [1] gate|up|down block
+    int I, T;
+    uint16_t *h;                  // [T, I]
+    uint16_t *y;                  // [T, H]
+};
+
+template <int BM, int BN, int BK, int SA, int SB>
+constexpr int kRingBytes = (SA * BM + SB * BN) * BK * 2;
+
 // Tile BM x BN x BK, WM x WN waves (4 or 8: with 8, two waves share each
 // SIMD so one wave's MFMAs cover the other's LDS reads, waits and
 // epilogue).  OCC is the number of workgroups per CU the tile is sized for
@@ -140,24 +162,6 @@ __device__ __forceinline__ void wait_stage(int younger) {
 // XCD b % 8): all n-tiles of an m-tile share the gathered activation rows
 // in one L2, and the m-tiles of one expert read the same weight tiles at
 // the same time from one L2.
-// Always-on shared experts as further tiles of a grouped launch (slot ==
-// nullptr: none): one MLP of intermediate I over rows 0 .. T-1 in order, on the
-// launch's own tile shape.  Its tiles take the first blocks of the grid: the
-// down half is the longest tile of the launch (K = shared I).  As launches of
-// their own on a second stream (48 blocks for the down half at T=1304) they
-// held CUs for long while the routed launches waited at the join, and their
-// time moved with how the two streams met (DeepSeek-V2-Lite layer, T=1304:
-// 320 to 360 us from run to run, 311 now; two layers of T=48 418 -> 398).
-struct SharedTiles {
-    const uint16_t *const *slot;  // [1] gate|up|down block
-    int I, T;
-    uint16_t *h;                  // [T, I]
-    uint16_t *y;                  // [T, H]
-};
-
-template <int BM, int BN, int BK, int SA, int SB>
-constexpr int kRingBytes = (SA * BM + SB * BN) * BK * 2;
-
 template <int BM, int BN, int BK, int WM, int WN, int SA, int SB, bool ILV, bool GATEUP, int OCC, int FK>
 __device__ __forceinline__ void grouped_tile(
     uint8_t *smem, const uint16_t *__restrict__ a_src, const int32_t *__restrict__ perm_token,
@@ -566,8 +570,11 @@ __global__ __launch_bounds__(64 * WM * WN, OCC == 1 ? 1 : OCC * WM * WN / 4) voi
 // either way, and the wider tile then reads their rows half as often.  Every
 // block compares the two m-tile counts of the same order, which the schedule
 // launch writes for both heights, and runs one body: 384 rows where they save
-// a quarter of the m-tiles or more.  Qwen shape, T=4096: uniform (128 tiles
-// against 190) 275 us on 384 rows, 280 on 256; Zipf 341 against 286.
+// a quarter of the m-tiles or more.  Both halves of the Qwen shape, T=4096:
+// uniform (128 tiles against 194) 444 us here, 438 on 384 rows alone and 447 on
+// 256; Zipf (178 against 218) 459, 495 and 458: two bodies in one kernel spill
+// 110 SGPRs, about 1% where the 384-row one runs (small layer, 94.9 against
+// 93.4), and the choice is worth 7% on the skewed routing.
 __global__ __launch_bounds__(512, 1) void grouped_gateup_pair_kernel(
     const uint16_t *__restrict__ x, const int32_t *__restrict__ perm_token, const int32_t *__restrict__ offsets,
     const int32_t *__restrict__ sel, int nsel, const int32_t *__restrict__ tile_start_384,

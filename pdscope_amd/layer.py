@@ -100,7 +100,7 @@ def decode_shared_fits(ws: MoEWorkspace) -> bool:
     """Whether one token with shared experts runs on the streaming GEMV
     kernels (three launches, no side stream) instead of the grouped ones
     (seven launches on two streams, whose 32-row tiles hold one row:
-    DeepSeek-V2-Lite shape, 82 us a layer against 34).  Only shapes that the
+    DeepSeek-V2-Lite shape, 85 us a layer against 33).  Only shapes that the
     grouped kernels take as well."""
     return (ws.H % 256 == 0 and ws.I % 128 == 0 and ws.shared_I % 64 == 0
             and ops.decode_shared_supported(ws.H, ws.I, ws.E, ws.k, ws.shared_I))
