@@ -74,7 +74,9 @@ __device__ __forceinline__ uint4 ld_nt(const void *p) {
 // scope): results no later block of the launch reads.  Plain stores stay in
 // the L2s, which write back what they hold while the kernel ends.  The two
 // wait states keep a VALU write to the data registers off a store that has not
-// read them yet (the compiler does not know of a store in an asm string).
+// read them yet (the compiler does not know of a store in an asm string).  Any
+// address is legal: the target runs in unaligned access mode, and the compiler
+// emits this instruction for a byte-aligned copy of 16 bytes too.
 __device__ __forceinline__ void st_through(void *p, uint4 v) {
     const u32x4_t d = {v.x, v.y, v.z, v.w};
     asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" ::"v"(p), "v"(d) : "memory");

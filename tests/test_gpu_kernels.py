@@ -729,3 +729,29 @@ def test_grouped_layer_tiles_equal_the_plain_launches(pd, T, bm, bmd, skew, shap
         assert torch.equal(h, ref_h) and torch.equal(y, ref_y)
         if with_shared:
             assert torch.equal(hs, ref_hs) and torch.equal(ys, ref_ys)
+
+
+@pytest.mark.parametrize("shift", [1, 3])
+def test_grouped_results_at_any_element_offset(pd, shift):
+    """y may start at any element of its storage (the tiles leave in 16-byte
+    stores): same bits as in an aligned buffer, nothing written around it."""
+    ops, layer, synthetic = pd
+    H, I, E, k, T = 256, 128, 32, 4, 70
+    lay = synthetic.make_layer(H, I, E, k, True, seed=8, device=DEV)
+    x = synthetic.make_tokens(T, H, seed=9, device=DEV)
+    slots = ops.slot_table([lay.experts[e] for e in range(E)], DEV)
+    ws = layer.MoEWorkspace(T, H, I, E, k, DEV)
+    _, ids, _ = layer.route(x, lay.gate, ws)
+    n = T * k
+    packed = ops.pack(ids, E)
+    sel = torch.arange(E, dtype=torch.int32, device=DEV)
+    for bm in (32, 64, 128, 256, 384):
+        order = torch.empty_like(sel)
+        ts, mt = ops.schedule(packed.counts, sel, bm, order=order), (n + bm - 1) // bm + E
+        bufs = [torch.full((n * H + 8,), 7.0, dtype=torch.bfloat16, device=DEV) for _ in range(2)]
+        views = bufs[0][:n * H], bufs[1][shift:shift + n * H]
+        for y in views:
+            ops.swiglu_grouped(x, packed.perm_token, packed.offsets, order, ts, mt, bm, slots, H, I, ws.h_ws, y)
+        torch.cuda.synchronize()
+        assert torch.equal(*views), bm
+        assert bool((bufs[1][:shift] == 7).all()) and bool((bufs[1][shift + n * H:] == 7).all())
